@@ -732,6 +732,22 @@ int pl_linear_shuffled(const void* x, int64_t ldx, int num_tokens,
                        int64_t ldo, int dtype, void* stream);
 
 /*
+ * pl_linear_shuffled for any number of tokens (prefill segments, large
+ * decode batches).  workspace (nullable, 16-byte aligned) of
+ * pl_linear_shuffled_wide_workspace_size bytes lets a call of few tokens
+ * split K over more workgroups; without it the call runs unsplit.  fp32
+ * accumulation, one rounding.  No counterpart in the reference: its base
+ * F.linear (model/flashinfer/packed_ops.py:143, 179, 251-265) at prefill
+ * sizes.
+ */
+size_t pl_linear_shuffled_wide_workspace_size(int num_tokens, int in_features, int out_features);
+int pl_linear_shuffled_wide(const void* x, int64_t ldx, int num_tokens,
+                            int in_features, const void* shuffled,
+                            int out_features, const void* bias, void* out,
+                            int64_t ldo, void* workspace,
+                            size_t workspace_bytes, int dtype, void* stream);
+
+/*
  * pl_linear_shuffled with K split over `splits` workgroups per 16-column
  * block: workgroup s sums k in [s*K/splits, (s+1)*K/splits) (whole 32-wide
  * steps) and writes fp32 plane s of partials (row t at t * ld, planes

@@ -42,6 +42,7 @@ _MFMA_VGPR = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 FILE_FLAGS = {
     "paged_prefill.hip": _MFMA_VGPR,
     "lora.hip": _MFMA_VGPR,
+    "wide_gemm.hip": _MFMA_VGPR,
 }
 
 

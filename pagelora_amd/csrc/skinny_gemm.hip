@@ -28,6 +28,7 @@
 
 #include "lora_up.h"
 #include "pl_common.h"
+#include "wide_gemm.h"
 
 namespace pl {
 namespace sgemm {
@@ -750,6 +751,12 @@ extern "C" int pl_linear_shuffled(const void* x, int64_t ldx, int num_tokens, in
   if (ldo < out_features) return fail(PL_ERR_INVALID, "ldo < out_features");
   if (dtype != PL_DTYPE_BF16 && dtype != PL_DTYPE_F16)
     return fail(PL_ERR_UNSUPPORTED, "pl_linear_shuffled dtype must be F16 or BF16 (got %d)", dtype);
+  // past one 16-token tile this kernel would stream W once per tile
+  if (num_tokens > 16 && wgemm::wide_supports(ldx)) {
+    const int st = wgemm::wide_linear(x, ldx, num_tokens, in_features, shuffled, out_features, bias, out, ldo, nullptr,
+                                      0, dtype, (hipStream_t)stream);
+    return st ? st : ok();
+  }
   const dim3 grid((out_features + 15) / 16, (num_tokens + 15) / 16);
   hipStream_t s = (hipStream_t)stream;
   if (dtype == PL_DTYPE_BF16)

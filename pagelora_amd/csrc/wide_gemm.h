@@ -1,0 +1,38 @@
+// Arguments and the host entry of the GEMM on shuffled weights past decode's
+// 16 tokens (wide_gemm.hip).
+#pragma once
+
+#include "pl_common.h"
+
+namespace pl {
+namespace wgemm {
+
+struct StripArgs {
+  const void* x;
+  const void* W;
+  const void* bias;
+  void* out;
+  int64_t ldx, ldo;
+  int tokens, K, N, m_tiles;
+};
+
+struct TileArgs {
+  const void* x;
+  const void* W;
+  const void* bias;
+  void* out;
+  float* partial;  // splits > 1: planes [splits][tokens][ldp]
+  int64_t ldx, ldo, ldp;
+  int tokens, K, N, m_tiles, n_tiles, splits, vec_out;
+};
+
+// 32-bit byte offsets reach every row of a token tile.
+bool wide_supports(int64_t ldx);
+
+// out = x . W^T (+ bias); arguments checked by the caller.  ws (nullable)
+// holds a K split's planes where one pays.
+int wide_linear(const void* x, int64_t ldx, int tokens, int K, const void* W, int N, const void* bias, void* out,
+                int64_t ldo, void* ws, size_t ws_bytes, int dtype, hipStream_t s);
+
+}  // namespace wgemm
+}  // namespace pl

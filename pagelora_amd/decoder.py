@@ -24,9 +24,9 @@ rides in the base GEMM (the adapters' A rows stacked under W) and the
 expand in the kernel that consumes the module output; o_proj's shrink runs
 in the attention's merge and down_proj's in SiLU*up, so no separate LoRA
 launches remain.  (With the fusion off, or past 16 rows: two add+RMSNorm
-kernels and the o/down GEMMs with their A rows on side planes, nine.)  Prefill, and batches beyond
-the decode GEMM's 64 rows, use the library GEMM (torch -> hipBLASLt);
-prefill forms q and appends k/v in the separate q/k norm + RoPE + append
+kernels and the o/down GEMMs with their A rows on side planes, nine.)  Past 16 rows (large decode
+batches, prefill) the same shuffled weights go through the tiled GEMM
+(linear_shuffled_wide); prefill forms q and appends k/v in the separate q/k norm + RoPE + append
 kernel.  Weights are random (no checkpoints are available); shapes follow
 Qwen3-8B.
 
@@ -44,7 +44,8 @@ from . import _lib, fused_ops
 from .attention_backend import PagedDecodeAttention
 from .kv_pool import PagedKVPool, Request
 from .linear import (LoraPartials, ShuffledWeight, SplitOutput, linear_shuffled, linear_shuffled_add,
-                     linear_shuffled_norm, linear_shuffled_side, linear_shuffled_split, lora_a_rows)
+                     linear_shuffled_norm, linear_shuffled_side, linear_shuffled_split, linear_shuffled_wide,
+                     lora_a_rows)
 from .lora import lora_linear
 
 
@@ -224,9 +225,8 @@ class LayerWeights:
         Unless ``keep_row_major``, the shuffled copy becomes the only one:
         the row-major [W; A] buffers are released (the LoRA A stacks move to
         tensors of their own), so the projection weights are stored once.
-        ``w_*_ext`` / ``w_*`` then return an unshuffled copy, and the library
-        GEMMs of prefill read the weight unshuffled into one buffer reused by
-        every projection (:func:`row_major`)."""
+        ``w_*_ext`` / ``w_*`` then return an unshuffled copy; the GEMMs of
+        decode and prefill read the shuffled one."""
         for name in ("qkv", "o", "gate_up", "down"):
             self.shuffled[name] = ShuffledWeight(getattr(self, f"w_{name}_ext"))
         if not keep_row_major:
@@ -317,8 +317,7 @@ class DecoderWeights:
     given (:meth:`from_tensors`).  ``shuffle`` (default) also builds the
     shuffled decode-GEMM copies of every projection and of the lm_head; the
     projections' row-major weights are then released unless
-    ``keep_row_major`` (the lm_head stays row-major too: prefill's last-token
-    logits and decode steps of more than 16 rows read it).
+    ``keep_row_major`` (the lm_head stays row-major too).
 
     ``adapter_version`` changes whenever the adapter stacks are reallocated
     (:meth:`set_adapter` past the stacked slots); decode graphs key on it, as
@@ -357,13 +356,11 @@ class DecoderWeights:
         return self._lm_head if self._lm_head is not None else self.lm_head_shuffled.unshuffle()
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
-        """x . lm_head^T: the shuffled GEMM at decode sizes (up to 16 rows, or
-        64 when no row-major copy is kept), else the library GEMM on the
-        row-major weight."""
-        limit = _lib.PL_LINEAR_MAX_TOKENS if self._lm_head is None else DECODE_GEMM_MAX_TOKENS
-        if self.lm_head_shuffled is not None and x.shape[0] <= limit:
-            return linear_shuffled(x, self.lm_head_shuffled)
-        return F.linear(x, self._lm_head if self._lm_head is not None else unshuffled_scratch(self.lm_head_shuffled))
+        """x . lm_head^T: the shuffled GEMM where that copy was made, else the
+        library GEMM on the row-major weight."""
+        if self.lm_head_shuffled is not None:
+            return linear_shuffled_wide(x, self.lm_head_shuffled)
+        return F.linear(x, self._lm_head)
 
     @classmethod
     def from_tensors(cls, cfg: DecoderConfig, *, embed: torch.Tensor, final_norm: torch.Tensor,
@@ -441,10 +438,10 @@ class DecodeContext:
         self.rope_cos_sin: torch.Tensor | None = None
 
 
-# Decode-sized inputs (up to 16 tokens) take the GEMM on shuffled weights
-# when the layer has them, else the row-major decode-sized linear kernel for
-# the narrow projections (q/k/v, o); the wide MLP projections and longer
-# inputs (prefill) take the library GEMM (torch -> hipBLASLt).
+# Layers with shuffled weights take the decode GEMM up to 16 tokens and the
+# tiled one past them.  Without: the row-major decode-sized linear kernel for
+# the narrow projections (q/k/v, o) up to 16 tokens, the library GEMM (torch
+# -> hipBLASLt) for the rest.
 DECODE_GEMM_MAX_TOKENS = 16
 # Split-K ways of the decode GEMM per projection (whole output, consumers
 # sum the planes).  None by default: down_proj ran split 3 ways (257 blocks
@@ -507,11 +504,10 @@ def _project(x: torch.Tensor, lw: LayerWeights, name: str) -> "torch.Tensor | Sp
     """x . [W; A]^T: the base output and every adapter's LoRA intermediate
     (at decode batch sizes as split-K planes, or with the intermediates split
     off, for the narrow projections)."""
-    # a single-copy layer keeps the shuffled GEMM up to 64 rows: unshuffling
-    # for the library GEMM would read the weight twice
-    limit = _lib.PL_LINEAR_MAX_TOKENS if lw.single_copy else DECODE_GEMM_MAX_TOKENS
-    if x.shape[0] <= limit:
-        sw = lw.shuffled.get(name)
+    sw = lw.shuffled.get(name)
+    if sw is not None and x.shape[0] > DECODE_GEMM_MAX_TOKENS:
+        return linear_shuffled_wide(x, sw)
+    if x.shape[0] <= DECODE_GEMM_MAX_TOKENS:
         if sw is not None:
             side = min(DECODE_SIDE_SPLITS.get(name, 0), sw.in_features // 32)
             main = lw.y_offset.get(name, sw.out_features)

@@ -95,21 +95,35 @@ class ShuffledWeight:
 def linear_shuffled(x: torch.Tensor, weight: ShuffledWeight, bias: torch.Tensor | None = None,
                     out: torch.Tensor | None = None) -> torch.Tensor:
     """``x . W^T (+ bias)`` for up to 64 tokens from a :class:`ShuffledWeight`."""
+    if x.dim() == 2 and x.shape[0] > _lib.PL_LINEAR_MAX_TOKENS:
+        raise ValueError(f"linear_shuffled takes at most {_lib.PL_LINEAR_MAX_TOKENS} tokens")
+    return linear_shuffled_wide(x, weight, bias, out)
+
+
+def linear_shuffled_wide(x: torch.Tensor, weight: ShuffledWeight, bias: torch.Tensor | None = None,
+                         out: torch.Tensor | None = None) -> torch.Tensor:
+    """``x . W^T (+ bias)`` for any number of tokens from a :class:`ShuffledWeight`."""
     if x.dim() != 2 or x.stride(1) != 1 or x.shape[1] != weight.in_features or x.dtype != weight.dtype:
         raise ValueError(f"x must be [T, {weight.in_features}] of {weight.dtype} with unit column stride")
-    T, N = x.shape[0], weight.out_features
-    if T > _lib.PL_LINEAR_MAX_TOKENS:
-        raise ValueError(f"linear_shuffled takes at most {_lib.PL_LINEAR_MAX_TOKENS} tokens")
+    T, K, N = x.shape[0], weight.in_features, weight.out_features
     out = torch.empty((T, N), dtype=x.dtype, device=x.device) if out is None else out
     if out.shape != (T, N) or out.stride(1) != 1 or out.dtype != x.dtype:
         raise ValueError("out must be [T, out] with unit column stride")
     if bias is not None and (bias.numel() != N or bias.dtype != x.dtype):
         raise ValueError("bias must be [out] of x's dtype")
     lib = _lib.load()
-    _lib.check(lib.pl_linear_shuffled(x.data_ptr(), x.stride(0), T, weight.in_features, weight.data.data_ptr(), N,
-                                      bias.data_ptr() if bias is not None else None, out.data_ptr(), out.stride(0),
-                                      _lib.dtype_code(x.dtype), _lib.stream_handle(x.device)),
-               "pl_linear_shuffled")
+    bias_ptr = bias.data_ptr() if bias is not None else None
+    if T <= 16:
+        _lib.check(lib.pl_linear_shuffled(x.data_ptr(), x.stride(0), T, K, weight.data.data_ptr(), N, bias_ptr,
+                                          out.data_ptr(), out.stride(0), _lib.dtype_code(x.dtype),
+                                          _lib.stream_handle(x.device)), "pl_linear_shuffled")
+        return out
+    nbytes = lib.pl_linear_shuffled_wide_workspace_size(T, K, N)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
+    _lib.check(lib.pl_linear_shuffled_wide(x.data_ptr(), x.stride(0), T, K, weight.data.data_ptr(), N, bias_ptr,
+                                           out.data_ptr(), out.stride(0), ws.data_ptr() if nbytes else None, nbytes,
+                                           _lib.dtype_code(x.dtype), _lib.stream_handle(x.device)),
+               "pl_linear_shuffled_wide")
     return out
 
 

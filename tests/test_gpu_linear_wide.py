@@ -1,0 +1,65 @@
+"""The GEMM on shuffled weights past 16 tokens (pl_linear_shuffled_wide) vs
+the oracle's linear term in float64: one rounding of the output (2^-8
+relative for bf16, 2^-11 for fp16) plus the fp32 accumulation's error, 2e-3
+max-abs, as for pl_linear_shuffled."""
+
+import numpy as np
+import pytest
+import torch
+
+from pagelora_amd import _lib
+from pagelora_amd.linear import ShuffledWeight, linear_shuffled_wide
+
+pytestmark = pytest.mark.gpu
+
+REL = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}
+
+
+# Edges of the token tiles (32 .. 256 rows), of the column tiles (128 .. 384)
+# and of the K steps: 64-wide ones fewer than the buffers in flight, K not a
+# multiple of 64 (the strip kernel), K split over workgroups (few tokens, wide
+# K), the tile shapes of many tokens.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,n,k", [
+    (17, 4112, 4096), (32, 1000, 96), (33, 6192, 64), (48, 24608, 192), (49, 37, 320), (64, 4112, 12288),
+    (65, 1000, 4096), (77, 4112, 4096), (81, 24608, 128), (100, 130, 224), (129, 2064, 4096), (191, 6192, 2048),
+    (257, 4112, 1024), (513, 24608, 256), (1000, 6192, 448), (2111, 4112, 320), (2112, 24608, 128),
+    (2200, 6192, 256), (2113, 24600, 64)])
+def test_linear_wide_vs_oracle(gpu_device, dtype, tokens, n, k):
+    print(f"[wide gemm] {tokens} x {n} x {k} {dtype}", flush=True)
+    g = torch.Generator(device=gpu_device).manual_seed(n + k + tokens)
+    x = torch.randn((tokens, k), generator=g, device=gpu_device).to(dtype)
+    w = (torch.randn((n, k), generator=g, device=gpu_device) * k ** -0.5).to(dtype)
+    bias = (torch.randn(n, generator=g, device=gpu_device) * 0.1).to(dtype) if tokens % 2 else None
+    sw = ShuffledWeight(w)
+    wide = torch.full((tokens, n + 9), 7.0, dtype=dtype, device=gpu_device)  # odd row stride, neighbours kept
+    out = linear_shuffled_wide(x, sw, bias, out=wide[:, :n])
+    whole = linear_shuffled_wide(x, sw, bias)
+    torch.cuda.synchronize()
+    assert torch.equal(out, whole) and (wide[:, n:] == 7.0).all()
+    want = x.double().cpu().numpy() @ w.double().cpu().numpy().T
+    if bias is not None:
+        want = want + bias.double().cpu().numpy()
+    err = np.abs(whole.float().cpu().numpy() - want)
+    assert (err <= 2e-3 + REL[dtype] * np.abs(want)).all(), f"max err {err.max():.3e}"
+
+
+def test_strided_x_without_workspace(gpu_device):
+    """x as a column slice of a wider buffer; no workspace: the same product
+    with its K sums in one piece."""
+    g = torch.Generator(device=gpu_device).manual_seed(5)
+    big = torch.randn((77, 4096 + 64), generator=g, device=gpu_device).to(torch.bfloat16)
+    w = (torch.randn((4112, 4096), generator=g, device=gpu_device) * 0.02).to(torch.bfloat16)
+    sw, lib = ShuffledWeight(w), _lib.load()
+    x = big[:, 64:]
+    assert lib.pl_linear_shuffled_wide_workspace_size(77, 4096, 4112) > 0
+    out = torch.empty((77, 4112), dtype=torch.bfloat16, device=gpu_device)
+    _lib.check(lib.pl_linear_shuffled_wide(x.data_ptr(), x.stride(0), 77, 4096, sw.data.data_ptr(), 4112, None,
+                                           out.data_ptr(), 4112, None, 0, _lib.dtype_code(x.dtype),
+                                           _lib.stream_handle(x.device)), "pl_linear_shuffled_wide")
+    split = linear_shuffled_wide(x, sw)
+    torch.cuda.synchronize()
+    want = x.double().cpu().numpy() @ w.double().cpu().numpy().T
+    for got in (out, split):
+        err = np.abs(got.float().cpu().numpy() - want)
+        assert (err <= 2e-3 + 2.0**-8 * np.abs(want)).all(), f"max err {err.max():.3e}"
