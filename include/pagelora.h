@@ -276,6 +276,42 @@ int pl_prefill_run(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                    int num_kv_heads, int head_dim, int page_size, int causal,
                    float sm_scale, int dtype, void* stream);
 
+/*
+ * The same plan for pl_prefill_split_run (head_dim 128, page_size a multiple
+ * of 4): records of eight int32, first the items (128 rows of a request over a
+ * range of 64-token kv tiles, the ranges cut where the rows alone would leave
+ * the GPU idle), then the merges of the row items that were cut.  Checks and
+ * errors as for pl_prefill_plan; *workspace_bytes_h receives the scratch a run
+ * needs (0 when nothing was cut).  PL_ERR_WORKSPACE if more than max_records
+ * records are needed.
+ */
+int pl_prefill_split_plan(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
+                          const int32_t* kv_last_page_len_h, int batch,
+                          int num_qo_heads, int num_kv_heads, int page_size,
+                          int causal, int32_t* items_h, int max_records,
+                          int* num_items_h, int* num_merges_h,
+                          size_t* workspace_bytes_h);
+
+/*
+ * pl_prefill_run over a plan of pl_prefill_split_plan: the same operation,
+ * arguments and checks at head_dim 128.  workspace (16-byte aligned, at least
+ * the plan's bytes; nullable when that is 0) holds the cut items' partial
+ * results during the call: calls that may run at the same time need one each.
+ */
+int pl_prefill_split_run(const void* q, int64_t q_stride_t, int64_t q_stride_h,
+                         const void* k_cache, const void* v_cache,
+                         int64_t page_stride, int64_t token_stride,
+                         int64_t head_stride, int64_t num_pages,
+                         const int32_t* qo_indptr, const int32_t* kv_indptr,
+                         const int32_t* kv_indices,
+                         const int32_t* kv_last_page_len, const int32_t* items,
+                         int num_items, int num_merges, void* o,
+                         int64_t o_stride_t, int64_t o_stride_h, int batch,
+                         int num_qo_heads, int num_kv_heads, int page_size,
+                         int causal, float sm_scale, void* workspace,
+                         size_t workspace_bytes, size_t plan_workspace_bytes,
+                         int dtype, void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Fused element-wise ops of the decode layer                                */
 /* ------------------------------------------------------------------------ */

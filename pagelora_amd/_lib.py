@@ -222,6 +222,29 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
             _f32, _i32, _vp,             # sm_scale, dtype, stream
         ],
     ),
+    "pl_prefill_split_plan": (
+        _i32,
+        [
+            _vp, _vp, _vp, _i32,         # qo_indptr, kv_indptr, last_page_len (host), batch
+            _i32, _i32, _i32, _i32,      # hq, hkv, page_size, causal
+            _vp, _i32,                   # records (host), max_records
+            ctypes.POINTER(_i32), ctypes.POINTER(_i32), ctypes.POINTER(_sz),  # num_items, num_merges, workspace bytes
+        ],
+    ),
+    "pl_prefill_split_run": (
+        _i32,
+        [
+            _vp, _i64, _i64,             # q, strides
+            _vp, _vp, _i64, _i64, _i64,  # k/v cache, page/token/head strides
+            _i64,                        # num_pages
+            _vp, _vp, _vp, _vp,          # qo_indptr, kv_indptr, kv_indices, last_page_len
+            _vp, _i32, _i32,             # records, num_items, num_merges
+            _vp, _i64, _i64,             # o, strides
+            _i32, _i32, _i32, _i32, _i32,  # batch, hq, hkv, page_size, causal
+            _f32, _vp, _sz, _sz,         # sm_scale, workspace, its bytes, the plan's bytes
+            _i32, _vp,                   # dtype, stream
+        ],
+    ),
     "pl_rmsnorm": (_i32, [_vp, _i64, _vp, _vp, _i64, _i32, _i32, _f32, _i32, _vp]),
     "pl_add_rmsnorm_lora": (
         _i32,

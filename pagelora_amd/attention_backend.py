@@ -577,17 +577,32 @@ class PagedDecodeAttention:
         max_page = _validate_host_table(kv_h, ind_h, last_h, self.page_size)
         if self.device.type != "cuda":
             raise RuntimeError("PagedDecodeAttention.plan_prefill needs a ROCm device")
-        n = ctypes.c_int(0)
+        n, merges, ws_bytes = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_size_t(0)
         args = (qo_h.data_ptr(), kv_h.data_ptr(), last_h.data_ptr(), batch, self.num_qo_heads, self.num_kv_heads,
                 self.page_size, int(bool(causal)))
-        _lib.check(self._lib.pl_prefill_plan(*args, None, 0, ctypes.byref(n)), "pl_prefill_plan")
-        items_h = torch.empty(max(1, 2 * n.value), dtype=torch.int32)
-        _lib.check(self._lib.pl_prefill_plan(*args, items_h.data_ptr(), n.value, ctypes.byref(n)), "pl_prefill_plan")
+        # the split-range kernel is built for head_dim 128 and loads four
+        # tokens of a page at a time; the 64-row kernel takes the rest
+        split = self.head_dim == 128 and self.page_size % 4 == 0
+        if split:
+            counts = (ctypes.byref(n), ctypes.byref(merges), ctypes.byref(ws_bytes))
+            _lib.check(self._lib.pl_prefill_split_plan(*args, None, 0, *counts), "pl_prefill_split_plan")
+            records = n.value + merges.value
+            items_h = torch.empty(max(1, 8 * records), dtype=torch.int32)
+            _lib.check(self._lib.pl_prefill_split_plan(*args, items_h.data_ptr(), records, *counts),
+                       "pl_prefill_split_plan")
+        else:
+            _lib.check(self._lib.pl_prefill_plan(*args, None, 0, ctypes.byref(n)), "pl_prefill_plan")
+            items_h = torch.empty(max(1, 2 * n.value), dtype=torch.int32)
+            _lib.check(self._lib.pl_prefill_plan(*args, items_h.data_ptr(), n.value, ctypes.byref(n)),
+                       "pl_prefill_plan")
         dev = [t.to(self.device, non_blocking=False) for t in (qo_h, kv_h, ind_h, last_h, items_h)]
         self._prefill_plan = {
             "batch": batch,
             "tokens": int(qo_h[-1]) if batch else 0,
             "num_items": n.value,
+            "split": split,
+            "num_merges": merges.value,
+            "workspace_bytes": ws_bytes.value,
             "causal": bool(causal),
             "max_page": max_page,
             "tables": dev,
@@ -637,6 +652,23 @@ class PagedDecodeAttention:
         if plan["max_page"] >= num_pages:
             raise ValueError(f"page id {plan['max_page']} is outside the {num_pages}-page KV pool")
         qo_d, kv_d, ind_d, last_d, items_d = plan["tables"]
+        if plan["split"]:
+            # per call, from torch's allocator: calls on other streams share nothing
+            nbytes = plan["workspace_bytes"]
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+            status = self._lib.pl_prefill_split_run(
+                q.data_ptr(), q.stride(0), q.stride(1),
+                k.data_ptr(), v.data_ptr(), page_stride, token_stride, head_stride,
+                num_pages,
+                qo_d.data_ptr(), kv_d.data_ptr(), ind_d.data_ptr(), last_d.data_ptr(),
+                items_d.data_ptr(), plan["num_items"], plan["num_merges"],
+                out.data_ptr(), out.stride(0), out.stride(1),
+                plan["batch"], self.num_qo_heads, self.num_kv_heads, self.page_size,
+                int(plan["causal"]), self.sm_scale, ws.data_ptr() if nbytes else None, nbytes, nbytes,
+                _lib.dtype_code(q.dtype), _lib.stream_handle(q.device),
+            )
+            _lib.check(status, "pl_prefill_split_run")
+            return out
         status = self._lib.pl_prefill_run(
             q.data_ptr(), q.stride(0), q.stride(1),
             k.data_ptr(), v.data_ptr(), page_stride, token_stride, head_stride,

@@ -41,6 +41,7 @@ HIPCC_FLAGS = [
 _MFMA_VGPR = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 FILE_FLAGS = {
     "paged_prefill.hip": _MFMA_VGPR,
+    "paged_prefill_split.hip": _MFMA_VGPR,
     "lora.hip": _MFMA_VGPR,
     "wide_gemm.hip": _MFMA_VGPR,
 }

@@ -1,0 +1,70 @@
+"""The split-range prefill kernel (head_dim 128, page sizes of a multiple of 4)
+vs the float64 oracle where it can go wrong: 64-token tile and 128-row item
+edges, kv ranges cut into parts, GQA groups that straddle items, strided q and
+out, and junk in the pages' unused slots.  Bars as in test_gpu_prefill."""
+
+import pytest
+import torch
+
+from tests.test_gpu_prefill import _backend, _case, _check, _oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("page_size", [4, 12, 16, 64])
+@pytest.mark.parametrize("heads,qo_lens,kv_lens,causal", [
+    ((2, 2), [1, 63, 64, 65], [64, 63, 128, 4097], True),      # a part per few tiles beside short requests
+    ((7, 1), [19, 0, 40], [2100, 5, 1025], True),              # groups of 7 across 16- and 128-row edges
+    ((8, 2), [3, 130], [1500, 300], False),
+    ((4, 4), [300], [300], True),
+])
+def test_edges_vs_oracle(gpu_device, dtype, page_size, heads, qo_lens, kv_lens, causal):
+    hq, hkv = heads
+    case = _case(qo_lens, kv_lens, hq, hkv, 128, page_size, dtype, gpu_device, seed=hq + page_size)
+    be = _backend(case, hq, hkv, 128, page_size, gpu_device, causal)
+    assert be._prefill_plan["split"]
+    # what lies past a request's last token in its last page is no part of the result
+    cache, ip, ind, last = case["cache"].clone(), case["indptr"], case["indices"], case["last"]
+    for r in range(len(kv_lens)):
+        cache[ind[ip[r + 1] - 1].item(), :, last[r].item():] = float("nan")
+    out = torch.empty((case["q"].shape[0], hq + 1, 128), dtype=dtype, device=gpu_device)[:, 1:]
+    q = torch.empty_like(out)
+    q.copy_(case["q"])
+    be.run_prefill_into(q, cache, out)
+    torch.cuda.synchronize()
+    _check(out, _oracle(case, causal), dtype)
+
+
+def test_long_range_is_cut_and_equals_whole(gpu_device):
+    """77 queries behind 9000 tokens: parts of the kv range agree with the 64-row kernel's whole one."""
+    case = _case([77], [9077], 8, 2, 128, 16, torch.float16, gpu_device, seed=1)
+    be = _backend(case, 8, 2, 128, 16, gpu_device)
+    assert be._prefill_plan["num_merges"] > 0
+    out = be.run_prefill(case["q"], case["cache"])
+    torch.cuda.synchronize()
+    _check(out, _oracle(case), torch.float16)
+
+
+@pytest.mark.parametrize("scale", [-0.05, 0.0])
+def test_scale_sign(gpu_device, scale):
+    """A negative or zero softmax scale: the same as the 64-row kernel on pages of 2 tokens."""
+    case = _case([50], [200], 4, 2, 128, 16, torch.bfloat16, gpu_device, seed=2)
+    be = _backend(case, 4, 2, 128, 16, gpu_device)
+    be.sm_scale = scale
+    out = be.run_prefill(case["q"], case["cache"])
+    pages = case["indices"].long()
+    small = case["cache"].cpu()[pages]  # [pages, 2, 16, Hkv, D] -> pages of 2 tokens
+    small = small.reshape(len(pages), 2, 8, 2, 2, 128).transpose(1, 2).reshape(-1, 2, 2, 2, 128).contiguous()
+    from pagelora_amd.attention_backend import PagedDecodeAttention
+
+    ref = PagedDecodeAttention(device=gpu_device, workspace_mb=8, num_qo_heads=4, num_kv_heads=2, head_dim=128,
+                               page_size=2)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32)  # noqa: E731
+    ref.plan_prefill(qo_indptr=i32([0, 50]), paged_kv_indptr=i32([0, 100]),
+                     paged_kv_indices=torch.arange(100, dtype=torch.int32), paged_kv_last_page_len=i32([2]))
+    assert not ref._prefill_plan["split"]
+    ref.sm_scale = scale
+    want = ref.run_prefill(case["q"], small.to(gpu_device))
+    torch.cuda.synchronize()
+    _check(out, want.float().cpu().numpy(), torch.bfloat16)
