@@ -28,6 +28,7 @@
 
 #include "pl_common.h"
 #include "lora_up.h"
+#include "prompt_ops.h"
 
 namespace pl {
 namespace fused {
@@ -987,6 +988,11 @@ static int silu_common(const void* gate_up, int64_t ldg, void* out, int64_t ldo,
     rank = lg.rank;
   }
   hipStream_t s = (hipStream_t)stream;
+  if (rank > 0 && dtype != PL_DTYPE_F32 && prompt::takes(rows, lg) && rows <= 32 * 65535) {
+    prompt::silu_mul(gate_up, ldg, out, ldo, rows, inter, lg, lu, dtype == PL_DTYPE_BF16, s);
+    PL_LAUNCH_CHECK("silu_mul_tile_kernel");
+    return ok();
+  }
   switch (dtype) {
     case PL_DTYPE_F32: return launch_silu<float>(rank, s, gate_up, ldg, out, ldo, rows, inter, lg, lu, ids, n_adapters);
     case PL_DTYPE_F16: return launch_silu<f16_t>(rank, s, gate_up, ldg, out, ldo, rows, inter, lg, lu, ids, n_adapters);
@@ -1159,6 +1165,15 @@ static int qkr_common(const void* qkv, int64_t ld_qkv, const void* q_norm_weight
         return st;
     if (a.lora.m[1].rank != a.lora.m[0].rank || a.lora.m[2].rank != a.lora.m[0].rank)
       return fail(PL_ERR_UNSUPPORTED, "q, k and v LoRA ranks differ");
+    const prompt::QkrTileArgs t{qkv, q_norm_weight, k_norm_weight, ld_qkv, positions, page_id, offset, q_out, k_cache,
+                                v_cache, page_stride, token_stride, head_stride, num_pages, page_size, batch,
+                                num_qo_heads, num_kv_heads, inv_freq, eps,
+                                {a.lora.m[0], a.lora.m[1], a.lora.m[2]}};
+    if (xs.splits == 0 && dtype != PL_DTYPE_F32 && prompt::takes_qkr(t, head_dim) && batch <= 16 * 65535) {
+      prompt::qk_norm_rope_append(t, dtype == PL_DTYPE_BF16, (hipStream_t)stream);
+      PL_LAUNCH_CHECK("qkr_tile_kernel");
+      return ok();
+    }
     return qkr_by_dtype(dtype, a.lora.m[0].rank, head_dim, a, (hipStream_t)stream);
   }
   return qkr_by_dtype(dtype, 0, head_dim, a, (hipStream_t)stream);
