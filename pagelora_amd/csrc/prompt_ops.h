@@ -13,8 +13,8 @@ namespace prompt {
 // 256 26.5 -> 8.7, 2112 264 -> 40.
 constexpr int kMinRows = 24;
 // q/k norm + RoPE + append, 48 heads: 2112 rows 45 -> 21 us, 512 rows 16.8 ->
-// 13.9, but a tile's
-// chain of three heads costs 11 us where the row kernel takes 5.5 (77 rows).
+// 13.9, but a tile's chain of three heads costs 11 us where the row kernel
+// takes 5.5 (77 rows).
 constexpr int kMinQkrRows = 512;
 
 struct QkrTileArgs {

@@ -385,19 +385,25 @@ struct Choice {
   double us;
 };
 
-// The estimated time of every tile shape and K split, from timings on MI355X
-// (24608 / 6192 / 4112 outputs over K = 4096 and 12288, 48 .. 2112 tokens):
-// a workgroup alone on its CU takes 0.42 + 0.026 u us per 64-wide step of u =
-// mf * nf fragments per wave; with every CU busy a step costs 0.0485 u where
-// u >= 24 and 0.067 u below (two or more workgroups share the CU); the
-// weights stream at 5.3 TB/s; a split adds a launch and its planes' traffic.
+// The estimated time of every tile shape and K split, fitted to timings on
+// MI355X (ten weights of 1000 .. 24608 outputs over K = 1024 .. 12288, 33 ..
+// 2112 tokens; the shape taken is within 1.0 % of the fastest one in the
+// geometric mean): a workgroup alone on its CU takes 0.34 + 0.024 u us per
+// 64-wide step of u = mf * nf fragments per wave, plus four steps to fill and
+// drain its pipeline; with every CU busy a step costs its MFMAs, 0.0485 u
+// where u >= 24 and 0.067 u below, or its operands at the 52 KB/us that a CU
+// gets out of the L2 (16 nf KB of weights, which every further token tile
+// streams again, and 2 mf KB of x), whichever is more; the weights stream from
+// memory at 5.3 TB/s; a split adds a launch and its planes' traffic.  Without
+// the L2 term few tokens took tiles of 32 (77 x 24608 x 4096: 74 us, now 44).
 static Choice choose(int tokens, int N, int K, bool allow_split) {
   Choice best{0, 1, 1e30};
   const int steps = K / 64;
   for (int i = 0; i < kNumShapes; ++i) {
     const TileShape& s = kShapes[i];
     const int u = s.mf * s.nf;
-    const double alone = 0.42 + 0.026 * u, busy = (u >= 24 ? 0.0485 : 0.067) * u;
+    const double alone = 0.34 + 0.024 * u;
+    const double busy = std::max((u >= 24 ? 0.0485 : 0.067) * u, (16 * s.nf + 2 * s.mf) / 52.0);
     const int64_t tiles = (int64_t)((tokens + 16 * s.mf - 1) / (16 * s.mf)) * ((N + 128 * s.nf - 1) / (128 * s.nf));
     for (int sp = 1; sp <= (allow_split ? 8 : 1); sp *= 2) {
       if (sp > 1 && (steps < 4 * sp || (int64_t)tokens * N * sp > (int64_t)kMaxSplitCells)) break;
@@ -410,8 +416,8 @@ static Choice choose(int tokens, int N, int K, bool allow_split) {
         step_us = std::max(alone * std::ceil(r / s.per_cu), r > 1 ? std::ceil(r) * busy : 0.0);
       }
       const double mem = ((double)N * K * 2 + (double)tokens * K * 2) / 5.3e6;
-      double us = 4.0 + std::max(step_us * ((steps + sp - 1) / sp), mem);
-      if (sp > 1) us += 3.5 + (double)tokens * N * 8 * sp / 8e6;
+      double us = 4.0 + std::max(step_us * ((steps + sp - 1) / sp + 4), mem);
+      if (sp > 1) us += 4.5 + (double)tokens * N * 8 * sp / 8e6;
       if (us < best.us) best = Choice{i, sp, us};
     }
   }
