@@ -89,6 +89,21 @@ def _validate_host_table(indptr: torch.Tensor, indices: torch.Tensor, last: torc
     return int(used.max()) if used.numel() else -1
 
 
+def _upload_int32(host: "Sequence[torch.Tensor]", device: torch.device) -> list[torch.Tensor]:
+    """int32 host tensors as views of one device buffer, 16-byte aligned each:
+    one asynchronous copy on the current stream from pinned memory (torch's
+    pinned allocator keeps the block until the copy is done)."""
+    starts, total = [], 0
+    for t in host:
+        starts.append(total)
+        total += -(-t.numel() // 4) * 4
+    staging = torch.empty(max(total, 4), dtype=torch.int32, pin_memory=True)
+    for t, at in zip(host, starts):
+        staging[at:at + t.numel()] = t
+    buf = staging.to(device, non_blocking=True)
+    return [buf[at:at + t.numel()] for t, at in zip(host, starts)]
+
+
 def _cache_geometry(cache, num_kv_heads: int, head_dim: int, page_size: int):
     """(k_tensor, v_tensor_or_ptr_source, page_stride, token_stride, head_stride, num_pages)."""
 
@@ -563,7 +578,9 @@ class PagedDecodeAttention:
         ``qo_len`` positions of its paged sequence; with ``causal`` query j
         sees kv positions ``<= kv_len - qo_len + j``.  The work list is built
         on the host (the tables are read there, as FlashInfer's prefill plan
-        does), then tables and work list are uploaded on the current stream.
+        does), then tables and work list are uploaded on the current stream,
+        without waiting for it (five copies that each did held the GPU idle
+        for 260 us of a 77-token prefill's plan).
         """
 
         tables = (qo_indptr, paged_kv_indptr, paged_kv_indices, paged_kv_last_page_len)
@@ -595,7 +612,11 @@ class PagedDecodeAttention:
             items_h = torch.empty(max(1, 2 * n.value), dtype=torch.int32)
             _lib.check(self._lib.pl_prefill_plan(*args, items_h.data_ptr(), n.value, ctypes.byref(n)),
                        "pl_prefill_plan")
-        dev = [t.to(self.device, non_blocking=False) for t in (qo_h, kv_h, ind_h, last_h, items_h)]
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("plan_prefill uploads host tables and cannot be captured")
+        dev = _upload_int32((items_h, qo_h, kv_h, ind_h, last_h), self.device)
+        items_d, *tables_d = dev
+        stream = torch.cuda.current_stream(self.device)
         self._prefill_plan = {
             "batch": batch,
             "tokens": int(qo_h[-1]) if batch else 0,
@@ -605,7 +626,10 @@ class PagedDecodeAttention:
             "workspace_bytes": ws_bytes.value,
             "causal": bool(causal),
             "max_page": max_page,
-            "tables": dev,
+            "tables": (*tables_d, items_d),
+            # the upload is asynchronous: a run on another stream waits for it
+            "stream": stream,
+            "ready": stream.record_event(),
             "q_data_type": q_data_type,
             "kv_data_type": kv_data_type,
         }
@@ -652,6 +676,11 @@ class PagedDecodeAttention:
         if plan["max_page"] >= num_pages:
             raise ValueError(f"page id {plan['max_page']} is outside the {num_pages}-page KV pool")
         qo_d, kv_d, ind_d, last_d, items_d = plan["tables"]
+        stream = torch.cuda.current_stream(q.device)
+        if stream != plan["stream"] and not torch.cuda.is_current_stream_capturing():
+            # (a capture begins after a device synchronization, past the upload)
+            stream.wait_event(plan["ready"])
+            qo_d.record_stream(stream)  # one allocation holds every table
         if plan["split"]:
             # per call, from torch's allocator: calls on other streams share nothing
             nbytes = plan["workspace_bytes"]

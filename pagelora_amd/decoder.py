@@ -828,7 +828,7 @@ def prefill(weights: DecoderWeights, pool: PagedKVPool, request: Request, tokens
     start = request.length - tokens.numel()
     assert start >= 0, "reserve pages for the prompt before prefill"
     host_pages = request.pages()
-    pages = torch.tensor(host_pages, dtype=torch.int64, device=tokens.device)
+    pages = torch.tensor(host_pages, dtype=torch.int64)
     if backend is None:
         backend = prefill_backend(cfg, ps, tokens.device)
     s = weights.lora_scale
@@ -845,9 +845,14 @@ def prefill(weights: DecoderWeights, pool: PagedKVPool, request: Request, tokens
             paged_kv_last_page_len=torch.tensor([ctx_len - ps * (n_pages - 1)], dtype=torch.int32),
             causal=True,
         )
-        pos = torch.arange(start + c0, ctx_len, device=tokens.device)
-        page_of = pages[pos // ps]
-        off_of = pos % ps
+        # positions, pages and page offsets of the chunk's tokens: formed on
+        # the host, one asynchronous copy (on the device six small kernels
+        # behind a copy that waited)
+        slots = torch.empty((3, T), dtype=torch.int64, pin_memory=True)
+        torch.arange(start + c0, ctx_len, out=slots[0])
+        slots[1] = pages[slots[0] // ps]
+        slots[2] = slots[0] % ps
+        pos, page_of, off_of = slots.to(tokens.device, non_blocking=True)
         hidden = F.embedding(tok, weights.embed)
         ids = torch.full((T,), adapter, dtype=torch.int32, device=tokens.device)
         attn = torch.empty((T, cfg.num_qo_heads, cfg.head_dim), dtype=hidden.dtype, device=tokens.device)

@@ -68,3 +68,25 @@ def test_scale_sign(gpu_device, scale):
     want = ref.run_prefill(case["q"], small.to(gpu_device))
     torch.cuda.synchronize()
     _check(out, want.float().cpu().numpy(), torch.bfloat16)
+
+
+def test_run_on_another_stream_follows_the_plan(gpu_device):
+    """The plan's upload is asynchronous: a run on a stream of its own, right
+    after plan_prefill and behind pending work on the planning stream, reads
+    the plan's tables, and a later plan's upload does not disturb it."""
+    cases = [_case([77], [9077], 8, 2, 128, 16, torch.bfloat16, gpu_device, seed=s) for s in (1, 2)]
+    want = []
+    for c in cases:
+        want.append(_backend(c, 8, 2, 128, 16, gpu_device).run_prefill(c["q"], c["cache"]))
+    be = _backend(cases[0], 8, 2, 128, 16, gpu_device)
+    torch.cuda.synchronize()
+    side, got = torch.cuda.Stream(), []
+    big = torch.randn((4096, 4096), device=gpu_device)
+    for c in cases:
+        big = (big @ big).clamp_(-1, 1)  # the planning stream is busy when the upload is enqueued
+        be.plan_prefill(qo_indptr=c["qo_indptr"], paged_kv_indptr=c["indptr"], paged_kv_indices=c["indices"],
+                        paged_kv_last_page_len=c["last"])
+        with torch.cuda.stream(side):
+            got.append(be.run_prefill(c["q"], c["cache"]))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
