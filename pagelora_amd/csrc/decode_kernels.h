@@ -489,8 +489,140 @@ struct DecodeWaveMfma {
   }
 };
 
+// D += A . B on a 16x16x16 MFMA tile (four k elements per lane, two words).
+template <typename T> __device__ __forceinline__ f32x4 mfma_16x16x16(uint2 a, uint2 b, f32x4 c);
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
+template <> __device__ __forceinline__ f32x4 mfma_16x16x16<bf16_t>(uint2 a, uint2 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4_t, a), __builtin_bit_cast(i16x4_t, b), c,
+                                                   0, 0, 0);
+}
+template <> __device__ __forceinline__ f32x4 mfma_16x16x16<f16_t>(uint2 a, uint2 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4_t, a), __builtin_bit_cast(f16x4_t, b), c, 0, 0,
+                                               0);
+}
+
+// A probability pair as two planes of T: the value cut to T, and what the cut
+// left (bf16: 16 bits of the mantissa, fp16: 22).  Both planes stay above zero
+// (by T's least useful value), so an infinite V gives the infinity that the
+// product with the whole probability gives, not 0 * inf.
+template <typename T> struct PlanePair;
+template <> struct PlanePair<bf16_t> {
+  static constexpr float kTiny = 1.17549435e-38f;
+  static __device__ __forceinline__ uint32_t cut(float a, float b) {
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+  }
+};
+template <> struct PlanePair<f16_t> {
+  static constexpr float kTiny = 5.9604645e-8f;
+  static __device__ __forceinline__ uint32_t cut(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+  }
+};
+
+// The wave for GQA groups of 5 to 8 heads, head_dim 128, 16-bit types: scores
+// as in DecodeWaveMfma with a head in each of the 16 columns (those past the
+// group repeat its last head), and P . V on MFMA too, straight from the
+// layout the loads leave: lane l holds dims 8 (l % 16) .. +8 of tokens
+// l / 16 + 4 i, so dim d of the eight is a 16x16x16 tile's A operand (row
+// l % 16, k = (l / 16, i)) after two byte permutes, and the lane's scores are
+// those tokens' of head l % 16: the B operand.  DecodeWave spends 64 FMAs and
+// dot products per head and block instead: 23 ragged rows, 7 heads per kv
+// head, 52 us of VALU work for 106 MB.
 template <typename T, int D, int G>
-using WaveFor = std::conditional_t<D == 128 && G == 4 && sizeof(T) == 2, DecodeWaveMfma<T, D, G>, DecodeWave<T, D, G>>;
+struct DecodeWaveMatrix {
+  static_assert(D == 128 && G <= 16 && sizeof(T) == 2, "P . V on MFMA: head_dim 128, 16-bit");
+  static constexpr int LPT = D / 8;
+  static constexpr int TPI = kWave / LPT;
+  static constexpr int NS = kBlockTokens / TPI;
+  static constexpr int W = 4;
+  static constexpr bool kMfmaScores = true;
+  using L8 = Lane8<T>;
+  static_assert(NS == 4, "four token rows per lane: one k group of the 16x16x16 tile");
+
+  uint32_t qb[NS][W];  // B operand: head lane % 16, dims 32 j + 8 (lane / 16) ..
+  float mo, lo;        // head lane % 16: running max (all lane rows), sum of this lane row's tokens
+  f32x4 acc[8];        // acc[d][i]: dim 32 (lane / 16) + 8 i + d of head lane % 16
+
+  __device__ void init() {
+    mo = -INFINITY;
+    lo = 0.f;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  __device__ static int64_t k_lane_off(int lane, int64_t token_stride) {
+    return DecodeWaveMfma<T, D, 4>::k_lane_off(lane, token_stride);
+  }
+
+  template <bool MASK>
+  __device__ __forceinline__ void consume(const uint32_t (&kw)[NS][W], const uint32_t (&vw_in)[NS][W],
+                                          float scale_log2, int row, int valid) {
+    f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NS; ++j) sacc = mfma_16x16x32<T>(kw[j], qb[j], sacc);
+    float sc[NS], mx = -INFINITY;
+    uint32_t vw[NS][W];
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const bool ok = !MASK || row + i * TPI < valid;
+      sc[i] = ok ? sacc[i] * scale_log2 : -INFINITY;
+      mx = fmaxf(mx, sc[i]);
+#pragma unroll
+      for (int w = 0; w < W; ++w) vw[i][w] = ok ? vw_in[i][w] : 0u;
+    }
+    // the tiles sum over all four lane rows: one maximum per head
+    if (__builtin_amdgcn_ballot_w64(mx > mo) != 0) {
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float m_new = fmaxf(mo, mx);
+      const float alpha = fast_exp2(mo - (m_new == -INFINITY ? 0.f : m_new));
+      mo = m_new;
+      lo *= alpha;
+#pragma unroll
+      for (int d = 0; d < 8; ++d)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[d][i] *= alpha;
+    }
+    const float m_use = mo == -INFINITY ? 0.f : mo;
+    using PP = PlanePair<T>;
+    uint32_t hi[2], low[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      float p[2], h[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        p[e] = fast_exp2(sc[2 * k + e] - m_use);
+        lo += p[e];
+        p[e] = fmaxf(p[e], PP::kTiny) + (p[e] != p[e] ? p[e] : 0.f);  // (a NaN stays one)
+      }
+      hi[k] = PP::cut(p[0], p[1]);
+      unpack2<T>(hi[k], h[0], h[1]);
+      low[k] = pack2_hw<T>(fmaxf(p[0] - h[0], PP::kTiny), fmaxf(p[1] - h[1], PP::kTiny));
+    }
+    const uint2 bh = make_uint2(hi[0], hi[1]), bl = make_uint2(low[0], low[1]);
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      const uint32_t sel = d % 2 ? 0x07060302u : 0x05040100u;
+      const uint2 a = make_uint2(__builtin_amdgcn_perm(vw[1][d / 2], vw[0][d / 2], sel),
+                                 __builtin_amdgcn_perm(vw[3][d / 2], vw[2][d / 2], sel));
+      acc[d] = mfma_16x16x16<T>(a, bh, acc[d]);
+      acc[d] = mfma_16x16x16<T>(a, bl, acc[d]);
+    }
+  }
+
+  // lo: the head's whole sum
+  __device__ __forceinline__ void merge_rows() {
+    lo += __shfl_xor(lo, 16);
+    lo += __shfl_xor(lo, 32);
+  }
+};
+
+template <typename T, int D, int G>
+constexpr bool kMatrixWave = D == 128 && G >= 5 && sizeof(T) == 2;
+template <typename T, int D, int G>
+using WaveFor = std::conditional_t<D == 128 && G == 4 && sizeof(T) == 2, DecodeWaveMfma<T, D, G>,
+                                   std::conditional_t<kMatrixWave<T, D, G>, DecodeWaveMatrix<T, 128, G>,
+                                                      DecodeWave<T, D, G>>>;
 
 // Stream blocks [blk0, blk1) of an item (16 tokens each, the item's first
 // `ntok` tokens are real) through one wave's online-softmax state: each
@@ -1172,8 +1304,9 @@ __global__ __launch_bounds__(kWave * waves_per_wg<FUSED>()) void decode_kernel(
     head_base_load<T, R>(qin, b, (is_k ? num_qo_heads : num_qo_heads + num_kv_heads) + h, col,
                          is_k ? (const T*)qin.k_norm_w : nullptr, hkv_in);
   } else if constexpr (WaveT::kMfmaScores) {
-    // the B operand: head lane % 4 of the group, dims 32 j + 8 (lane / 16)
-    const T* qp = q + (int64_t)b * q_sb + (int64_t)(h * G + lane % 4) * q_sh + 8 * (lane / 16);
+    // the B operand: head lane % 4 (lane % 16) of the group, dims 32 j + 8 (lane / 16)
+    const int qg = kMatrixWave<T, D, G> ? min(lane % 16, G - 1) : lane % 4;
+    const T* qp = q + (int64_t)b * q_sb + (int64_t)(h * G + qg) * q_sh + 8 * (lane / 16);
 #pragma unroll
     for (int j = 0; j < WaveT::NS; ++j) L8::load(st.qb[j], qp + 32 * j);
   } else {
@@ -1315,6 +1448,29 @@ __global__ __launch_bounds__(kWave * waves_per_wg<FUSED>()) void decode_kernel(
   constexpr float kLn2 = 0.69314718055994530942f;
   bool direct = flags & 1;  // the row is one item: write the output directly
   if constexpr (FUSED) direct = direct && !qin.no_direct;
+  if constexpr (kMatrixWave<T, D, G>) {
+    // lane: head lane % 16, dims 32 (lane / 16) .. +32
+    const int g = lane % 16;
+    if (g >= G) return;
+    const int hq = h * G + g;
+    const float inv = st.lo > 0.f ? 1.f / st.lo : 0.f;
+    const int64_t slot_row = (int64_t)(flags >> 2) * num_qo_heads + hq;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int dim = 32 * row + 8 * i;
+      float out[8];
+#pragma unroll
+      for (int d = 0; d < 8; ++d) out[d] = st.acc[d][i] * inv;
+      if (direct)
+        L8::store(o + (int64_t)b * o_sb + (int64_t)hq * o_sh + dim, out);
+      else
+        Lane8<float>::store(part_o + slot_row * D + dim, out);
+    }
+    const float lse2 = st.lo > 0.f ? st.mo + __log2f(st.lo) : -INFINITY;  // log2
+    if (row == 0 && direct && lse != nullptr) lse[(int64_t)b * num_qo_heads + hq] = lse2 * kLn2;
+    if (row == 0 && !direct) part_lse[slot_row] = lse2;
+    return;
+  } else {
   if (direct) {
     if (row != 0) return;
 #pragma unroll
@@ -1348,6 +1504,7 @@ __global__ __launch_bounds__(kWave * waves_per_wg<FUSED>()) void decode_kernel(
       part_lse[(int64_t)slot * num_qo_heads + hq] =
           st.l[g] > 0.f ? st.m[g] + __log2f(st.l[g]) : -INFINITY;
   }
+  }  // !kMatrixWave
 }
 
 // ----------------------------------------------------------------- merge ---

@@ -17,6 +17,13 @@
 // (ds_read_b64_tr_b16) and serves both columns.  An item of a split range
 // leaves its unnormalized output and softmax state in the workspace, and
 // merge_kernel combines a row's parts in order.
+//
+// Bound by the matrix and vector units' shared issue: 8192 tokens of 32768
+// (GQA 4, bf16) 7885 us with 64-row items and 16 rows per wave -> 4490 us, the
+// MFMAs busy 58 % of the cycles (bf16's P is two planes, a third of them).
+// One wave's softmax beside its own neighbouring half tiles' MFMAs (software
+// pipelining) was slower (5190 us): two waves per SIMD overlap already, and
+// its registers spill.
 #include <algorithm>
 #include <type_traits>
 #include <vector>
@@ -107,6 +114,12 @@ struct Args {
 template <typename T, bool PAGE16>
 __global__ __launch_bounds__(kThreads, 2) void prefill_split_kernel(Args A) {
   constexpr int NPP = std::is_same<T, bf16_t>::value ? 2 : 1;  // P planes: hi (+ lo)
+  // A column's running maximum follows only scores more than this above it,
+  // which takes the rescale (64 multiplies and the lanes' exchange) out of
+  // the steady state.  P's two planes hold probabilities up to 2^8 as well as
+  // those up to 1; the one fp16 plane is exact for the largest only where
+  // that is 1 (2.6e-4 against 2.5e-4 with a lag, from 64 bits).
+  constexpr float kLag = NPP == 2 ? 8.f : 0.f;
   // one object per buffer: loads into one never alias reads of another
   __shared__ __align__(16) char s_k0[kBufBytes];
   __shared__ __align__(16) char s_v0[kBufBytes];
@@ -237,15 +250,24 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_split_kernel(Args A) {
     if (tile * kTile > lim_hi) return;  // (uniform) no row of the wave sees the tile
 
     f32x4 s[kCols][4];
+    // four independent accumulations in turn, here and below: an MFMA waits
+    // for the one before it on the same accumulator
 #pragma unroll
-    for (int blk = 0; blk < 4; ++blk) {
+    for (int b0 = 0; b0 < 4; b0 += 2) {
 #pragma unroll
-      for (int c = 0; c < kCols; ++c) s[c][blk] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < kCols; ++c)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) s[c][b0 + b] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        const u32x4 ka = *reinterpret_cast<const u32x4*>(kb + kaddr[ks] + blk * 16 * kRowBytes);
+        u32x4 ka[2];
 #pragma unroll
-        for (int c = 0; c < kCols; ++c) s[c][blk] = mfma32<T>(ka, qb[c][ks], s[c][blk]);
+        for (int b = 0; b < 2; ++b)
+          ka[b] = *reinterpret_cast<const u32x4*>(kb + kaddr[ks] + (b0 + b) * 16 * kRowBytes);
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int c = 0; c < kCols; ++c) s[c][b0 + b] = mfma32<T>(ka[b], qb[c][ks], s[c][b0 + b]);
       }
     }
     if (tile * kTile + kTile - 1 > lim_lo) {
@@ -267,10 +289,11 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_split_kernel(Args A) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) v = fmaxf(v, s[c][blk][i]);
       mx[c] = v * sc;
-      rose |= mx[c] > m[c];
+      rose |= mx[c] > m[c] + kLag;
     }
     // the columns' maxima are reduced over their lanes, and the sums and
-    // accumulators rescaled, only where some lane saw a larger score
+    // accumulators rescaled, only where some lane saw a score kLag past its
+    // maximum
     if (__builtin_amdgcn_ballot_w64(rose) != 0) {
 #pragma unroll
       for (int c = 0; c < kCols; ++c) {
@@ -317,14 +340,20 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_split_kernel(Args A) {
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-      for (int a = 0; a < 8; ++a) {
-        const u32x2 v0 = read_tr(vb + vaddr[a] + kc * 32 * kRowBytes);
-        const u32x2 v1 = read_tr(vb + vaddr[a] + (kc * 32 + 16) * kRowBytes);
-        const u32x4 va = {v0[0], v0[1], v1[0], v1[1]};
+      for (int a0 = 0; a0 < 8; a0 += 2) {
+        u32x4 va[2];
 #pragma unroll
-        for (int c = 0; c < kCols; ++c)
+        for (int a = 0; a < 2; ++a) {
+          const u32x2 v0 = read_tr(vb + vaddr[a0 + a] + kc * 32 * kRowBytes);
+          const u32x2 v1 = read_tr(vb + vaddr[a0 + a] + (kc * 32 + 16) * kRowBytes);
+          va[a] = u32x4{v0[0], v0[1], v1[0], v1[1]};
+        }
 #pragma unroll
-          for (int pl = 0; pl < NPP; ++pl) acc[c][a] = mfma32<T>(va, pb[c][kc][pl], acc[c][a]);
+        for (int pl = 0; pl < NPP; ++pl)
+#pragma unroll
+          for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int c = 0; c < kCols; ++c) acc[c][a0 + a] = mfma32<T>(va[a], pb[c][kc][pl], acc[c][a0 + a]);
       }
   };
 
@@ -385,17 +414,33 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(Args A, const Item* mer
   const int parts = uniform(it.parts);
   const float* p = A.part + ((int64_t)uniform(it.slot) * A.hkv + h) * kPartFloats;
   const int64_t step = (int64_t)A.hkv * kPartFloats;
+  // the parts' states one per lane, their outputs eight loads at a time
+  const float* ml = p + kRows * D + pr * 2;
   float top = -INFINITY;
-  for (int i = 0; i < parts; ++i) top = fmaxf(top, p[i * step + kRows * D + pr * 2]);
+  for (int b = lane; b < parts; b += kWave) top = fmaxf(top, ml[b * step]);
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) top = fmaxf(top, __shfl_xor(top, d));
   if (top == -INFINITY) top = 0.f;
   float sum = 0.f, o0 = 0.f, o1 = 0.f;
-  for (int i = 0; i < parts; ++i) {
-    const f32x2 ml = *reinterpret_cast<const f32x2*>(p + i * step + kRows * D + pr * 2);
-    const f32x2 v = *reinterpret_cast<const f32x2*>(p + i * step + pr * D + lane * 2);
-    const float w = fast_exp2(ml[0] - top);
-    sum += ml[1] * w;
-    o0 += v[0] * w;
-    o1 += v[1] * w;
+  for (int b0 = 0; b0 < parts; b0 += kWave) {
+    const int n = min(parts - b0, kWave);
+    const f32x2 own = lane < n ? *reinterpret_cast<const f32x2*>(ml + (b0 + lane) * step) : f32x2{-INFINITY, 0.f};
+    const float w = fast_exp2(own[0] - top);
+    const float lw = own[1] * w;
+    const float* q = p + b0 * step + pr * D + lane * 2;
+    for (int i0 = 0; i0 < n; i0 += 8) {
+      f32x2 v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const f32x2*>(q + min(i0 + i, n - 1) * step);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i0 + i >= n) break;
+        const float wi = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), i0 + i));
+        sum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(lw), i0 + i));
+        o0 = fmaf(v[i][0], wi, o0);
+        o1 = fmaf(v[i][1], wi, o1);
+      }
+    }
   }
   const float inv = sum > 0.f ? 1.f / sum : (sum == 0.f ? 0.f : sum);
   const int pos = row / g;
@@ -481,9 +526,11 @@ extern "C" int pl_prefill_split_plan(const int32_t* qo_indptr_h, const int32_t* 
   }
   if (list.size() > (size_t)INT32_MAX / 64) return fail(PL_ERR_INVALID, "too many prefill work items");
   // A part's length: an even share of the work per slot, if the longest row
-  // item is well past it (else the parts' traffic and the merge cost more).
+  // item is more than twice that (2119 tokens MHA, 1.7 times: 56.5 us whole,
+  // 68 cut; 77 behind 32000, 21 times: 77 us in 504 parts, 114 in 252, 87 in
+  // 1000).
   const int64_t share = std::max<int64_t>(kMinTiles, (work * num_kv_heads + kSlots - 1) / kSlots);
-  const int64_t chunk = longest > share + share / 2 ? share : INT32_MAX;
+  const int64_t chunk = longest > 2 * share ? share : INT32_MAX;
   std::vector<Item> items, merges;
   int slots = 0;
   for (const Rows& e : list) {
