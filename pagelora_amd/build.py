@@ -37,9 +37,12 @@ HIPCC_FLAGS = [
 # AGPRs.  paged_prefill: the softmax rescale then works on them in place (no
 # copies between the register files each tile) and the kernel needs 158
 # registers instead of 192 (three waves per SIMD instead of two).  lora: the
-# shrink kernel 72 -> 56 registers, the expand 72 -> 66.
+# shrink kernel 72 -> 56 registers, the expand 72 -> 66.  paged_decode: the
+# folded kernel's 255 + 32 registers fit 255, two waves per SIMD instead of one.
 _MFMA_VGPR = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 FILE_FLAGS = {
+    "paged_decode.hip": _MFMA_VGPR,
+    "paged_decode_small.hip": _MFMA_VGPR,
     "paged_prefill.hip": _MFMA_VGPR,
     "paged_prefill_split.hip": _MFMA_VGPR,
     "lora.hip": _MFMA_VGPR,

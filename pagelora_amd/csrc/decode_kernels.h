@@ -365,130 +365,6 @@ struct DecodeWave {
   __device__ __forceinline__ void merge_rows() { merge_lane_rows<G, LPT>(m, l, acc); }
 };
 
-// The score-on-MFMA wave for GQA groups of 4 heads, head_dim 128, 16-bit
-// types: per block of 16 tokens, S^T = K . Q^T is four
-// v_mfma_f32_16x16x32 (A: the block's K, lane l holding 8 dims of token
-// perm(l % 16); B: q, the group's 4 heads repeated over the 16 columns), in
-// place of 64 dot2 and 64 DPP reductions.  The token permutation
-// perm(m) = m / 4 + 4 * (m % 4) puts the scores of lane l's output rows
-// 4*(l/16) + i on tokens l/16 + 4i: the tokens whose V rows the lane already
-// holds in the VALU layout (row l/16, load s = i).  Lane l's scores are those
-// of head l % 4; each lane runs the online softmax of that head for its lane
-// row, and the quad's lanes (l & ~3 .. l | 3: heads 0..3 of the same tokens)
-// exchange p and the rescale factors with quad-permute DPP, so P . V stays
-// on VALU in registers as in DecodeWave.
-template <typename T, int D, int G>
-struct DecodeWaveMfma {
-  static_assert(D == 128 && G == 4 && sizeof(T) == 2, "MFMA scores: GQA 4, head_dim 128, 16-bit");
-  static constexpr int LPT = D / 8;             // V: lanes per token row
-  static constexpr int TPI = kWave / LPT;       // V: token rows per load instruction
-  static constexpr int NS = kBlockTokens / TPI; // loads per lane per block (K: one per 32 dims)
-  static constexpr int W = 4;
-  static constexpr bool kMfmaScores = true;
-  using L8 = Lane8<T>;
-
-  uint32_t qb[NS][W];  // B operand: head lane % 4, dims 32 j + 8 (lane / 16) ..
-  float mo, lo;        // online-softmax state of head lane % 4, lane row lane / 16 (log2)
-  float m[G], l[G];    // merge_rows: the state of every head
-  float acc[G][8];     // unnormalised output, this lane's 8 dims (8 * (lane % 16))
-
-  __device__ void init() {
-    mo = -INFINITY;
-    lo = 0.f;
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[g][i] = 0.f;
-  }
-
-  // Element offset of lane `lane`'s K piece for load j = 0 within a block:
-  // token perm(lane % 16), dims 8 * (lane / 16); load j adds 32 dims.
-  __device__ static int64_t k_lane_off(int lane, int64_t token_stride) {
-    const int m16 = lane % 16;
-    return (int64_t)(m16 / 4 + 4 * (m16 % 4)) * token_stride + 8 * (lane / 16);
-  }
-  // Lane of the block that holds token t's K (its 4 loads hold dims 32 j +
-  // 8 * (lane / 16)): the lanes l with l % 16 == perm^-1(t).
-  __device__ static int k_lane_of(int t) { return 4 * (t % 4) + t / 4; }
-
-  template <int CTRL>
-  __device__ static float quad_bcast(float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, false));
-  }
-
-  template <bool MASK>
-  __device__ __forceinline__ void consume(const uint32_t (&kw)[NS][W], const uint32_t (&vw)[NS][W],
-                                          float scale_log2, int row, int valid) {
-    f32x4 sacc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < NS; ++j) sacc = mfma_16x16x32<T>(kw[j], qb[j], sacc);
-    float sc[NS];
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      sc[i] = sacc[i] * scale_log2;
-      if (MASK) sc[i] = (row + i * TPI < valid) ? sc[i] : -INFINITY;
-    }
-    float vf[NS][8];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      L8::to_f32(vw[s], vf[s]);
-      if (MASK) {
-        const bool ok = row + s * TPI < valid;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) vf[s][i] = ok ? vf[s][i] : 0.f;
-      }
-    }
-    float mx = sc[0];
-#pragma unroll
-    for (int i = 1; i < NS; ++i) mx = fmaxf(mx, sc[i]);
-    const float m_new = fmaxf(mo, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;  // all masked so far
-    const float alpha = fast_exp2(mo - m_use);
-    mo = m_new;
-    float p[NS], psum = 0.f;
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      p[i] = fast_exp2(sc[i] - m_use);
-      psum += p[i];
-    }
-    lo = lo * alpha + psum;
-    // quad_perm:[g,g,g,g]: lane 4k + g of the quad holds head g
-    float ag[G], pg[NS][G];
-    ag[0] = quad_bcast<0x00>(alpha);
-    ag[1] = quad_bcast<0x55>(alpha);
-    ag[2] = quad_bcast<0xAA>(alpha);
-    ag[3] = quad_bcast<0xFF>(alpha);
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      pg[i][0] = quad_bcast<0x00>(p[i]);
-      pg[i][1] = quad_bcast<0x55>(p[i]);
-      pg[i][2] = quad_bcast<0xAA>(p[i]);
-      pg[i][3] = quad_bcast<0xFF>(p[i]);
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int d = 0; d < 8; ++d) {
-        float a = acc[g][d] * ag[g];
-#pragma unroll
-        for (int i = 0; i < NS; ++i) a = fmaf(pg[i][g], vf[i][d], a);
-        acc[g][d] = a;
-      }
-  }
-
-  __device__ __forceinline__ void merge_rows() {
-    m[0] = quad_bcast<0x00>(mo);
-    m[1] = quad_bcast<0x55>(mo);
-    m[2] = quad_bcast<0xAA>(mo);
-    m[3] = quad_bcast<0xFF>(mo);
-    l[0] = quad_bcast<0x00>(lo);
-    l[1] = quad_bcast<0x55>(lo);
-    l[2] = quad_bcast<0xAA>(lo);
-    l[3] = quad_bcast<0xFF>(lo);
-    merge_lane_rows<G, LPT>(m, l, acc);
-  }
-};
-
 // D += A . B on a 16x16x16 MFMA tile (four k elements per lane, two words).
 template <typename T> __device__ __forceinline__ f32x4 mfma_16x16x16(uint2 a, uint2 b, f32x4 c);
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
@@ -520,15 +396,22 @@ template <> struct PlanePair<f16_t> {
   }
 };
 
-// The wave for GQA groups of 5 to 8 heads, head_dim 128, 16-bit types: scores
-// as in DecodeWaveMfma with a head in each of the 16 columns (those past the
-// group repeat its last head), and P . V on MFMA too, straight from the
-// layout the loads leave: lane l holds dims 8 (l % 16) .. +8 of tokens
-// l / 16 + 4 i, so dim d of the eight is a 16x16x16 tile's A operand (row
-// l % 16, k = (l / 16, i)) after two byte permutes, and the lane's scores are
-// those tokens' of head l % 16: the B operand.  DecodeWave spends 64 FMAs and
-// dot products per head and block instead: 23 ragged rows, 7 heads per kv
-// head, 52 us of VALU work for 106 MB.
+// The wave for GQA groups of 4 heads and more, head_dim 128, 16-bit types:
+// both products on MFMA, straight from registers.  Per block of 16 tokens
+// S^T = K . Q^T is four v_mfma_f32_16x16x32 (A: the block's K, lane l holding
+// 8 dims of token perm(l % 16); B: q, one head of the group per column, those
+// past the group repeating its heads).  perm(m) = m / 4 + 4 * (m % 4) puts the
+// scores of lane l's output rows 4*(l/16) + i on tokens l/16 + 4i, the tokens
+// whose V rows the lane holds (row l/16, load s = i).  So O^T += V^T P^T needs
+// no exchange either: lane l holds dims 8 (l % 16) .. +8 of its four tokens,
+// and dim d of the eight is a 16x16x16 tile's A operand (row l % 16, k =
+// (l / 16, i)) after two byte permutes, the lane's probabilities of head
+// l % 16 the B operand.  The VALU forms of the products cost 64 dot products,
+// DPP sums and FMAs per head and block: 23 ragged rows of 7 heads per kv head
+// 53.7 -> 30.0 us (106 MB); 4 heads, whose P . V alone was on the VALU: 1 x
+// 2048 11.3 -> 9.75 us, 4 x 2112 15.7 -> 13.5, 1 x 32000 32.7 -> 29.2, 64 x
+// 2048 98.5 -> 96.0, the four-layer decode step 429 -> 423 (with the
+// accumulators in VGPRs; in AGPRs 0.2 to 0.7 us slower).
 template <typename T, int D, int G>
 struct DecodeWaveMatrix {
   static_assert(D == 128 && G <= 16 && sizeof(T) == 2, "P . V on MFMA: head_dim 128, 16-bit");
@@ -550,9 +433,15 @@ struct DecodeWaveMatrix {
 #pragma unroll
     for (int d = 0; d < 8; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  // Element offset of lane `lane`'s K piece for load j = 0 within a block:
+  // token perm(lane % 16), dims 8 * (lane / 16); load j adds 32 dims.
   __device__ static int64_t k_lane_off(int lane, int64_t token_stride) {
-    return DecodeWaveMfma<T, D, 4>::k_lane_off(lane, token_stride);
+    const int m16 = lane % 16;
+    return (int64_t)(m16 / 4 + 4 * (m16 % 4)) * token_stride + 8 * (lane / 16);
   }
+  // Lane of the block that holds token t's K (its 4 loads hold dims 32 j +
+  // 8 * (lane / 16)): the lanes l with l % 16 == perm^-1(t).
+  __device__ static int k_lane_of(int t) { return 4 * (t % 4) + t / 4; }
 
   template <bool MASK>
   __device__ __forceinline__ void consume(const uint32_t (&kw)[NS][W], const uint32_t (&vw_in)[NS][W],
@@ -618,11 +507,9 @@ struct DecodeWaveMatrix {
 };
 
 template <typename T, int D, int G>
-constexpr bool kMatrixWave = D == 128 && G >= 5 && sizeof(T) == 2;
+constexpr bool kMatrixWave = D == 128 && G >= 4 && sizeof(T) == 2;
 template <typename T, int D, int G>
-using WaveFor = std::conditional_t<D == 128 && G == 4 && sizeof(T) == 2, DecodeWaveMfma<T, D, G>,
-                                   std::conditional_t<kMatrixWave<T, D, G>, DecodeWaveMatrix<T, 128, G>,
-                                                      DecodeWave<T, D, G>>>;
+using WaveFor = std::conditional_t<kMatrixWave<T, D, G>, DecodeWaveMatrix<T, 128, G>, DecodeWave<T, D, G>>;
 
 // Stream blocks [blk0, blk1) of an item (16 tokens each, the item's first
 // `ntok` tokens are real) through one wave's online-softmax state: each
@@ -1304,9 +1191,8 @@ __global__ __launch_bounds__(kWave * waves_per_wg<FUSED>()) void decode_kernel(
     head_base_load<T, R>(qin, b, (is_k ? num_qo_heads : num_qo_heads + num_kv_heads) + h, col,
                          is_k ? (const T*)qin.k_norm_w : nullptr, hkv_in);
   } else if constexpr (WaveT::kMfmaScores) {
-    // the B operand: head lane % 4 (lane % 16) of the group, dims 32 j + 8 (lane / 16)
-    const int qg = kMatrixWave<T, D, G> ? min(lane % 16, G - 1) : lane % 4;
-    const T* qp = q + (int64_t)b * q_sb + (int64_t)(h * G + qg) * q_sh + 8 * (lane / 16);
+    // the B operand: head lane % 16 of the group, dims 32 j + 8 (lane / 16)
+    const T* qp = q + (int64_t)b * q_sb + (int64_t)(h * G + min(lane % 16, G - 1)) * q_sh + 8 * (lane / 16);
 #pragma unroll
     for (int j = 0; j < WaveT::NS; ++j) L8::load(st.qb[j], qp + 32 * j);
   } else {

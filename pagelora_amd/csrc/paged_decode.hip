@@ -14,9 +14,10 @@
 //                  (16 lanes x 16 B cover one 128-dim token row, so one
 //                  dwordx4 load instruction reads 4 token rows), scores them
 //                  against the g query heads of the kv head with v_dot2 and
-//                  DPP row reductions (GQA 4 at head_dim 128 in 16-bit
-//                  types: on MFMA, DecodeWaveMfma), and keeps an online
-//                  softmax per lane row in fp32.  Rows with one item write
+//                  DPP row reductions (groups of 4 heads and more at head_dim
+//                  128 in 16-bit types: both products on MFMA,
+//                  DecodeWaveMatrix), and keeps an online softmax in fp32.
+//                  Rows with one item write
 //                  the output directly; split rows write (o, lse) partials.
 //   merge_kernel   one wavefront per (row, q head) of a split row: the
 //                  LSE-weighted sum of its partials.  A separate launch, so
