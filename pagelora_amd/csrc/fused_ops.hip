@@ -257,6 +257,8 @@ __device__ __forceinline__ void load8_planes(const SplitIn& sp, int64_t t, int c
 }
 
 constexpr int kRowNormMaxHidden = 8192;
+constexpr int kNormRows = 2;       // rows per workgroup of add_rmsnorm_rows_kernel
+constexpr int kNormRowsMin = 320;  // from these rows on
 
 // YS: the module's y comes from ys.splits fp32 side planes (the LoRA A rows
 // of pl_linear_shuffled_side, column y_offset + a*R of each plane): thread
@@ -375,6 +377,75 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = v[i] * rstd * wf[i];
   if (live) store_row8<T>(out + row * ldo + idx, v);
+}
+
+// The same for prompts bound to one adapter: a workgroup takes N rows with the
+// module's B in registers.  The row kernel reads B's 128 KB (hidden 4096, rank
+// 16) out of the L2 for every row, which bounds it past a few hundred rows:
+// 384 rows 6.1 -> 5.3 us, 1024 10.7 -> 9.1, 2112 21.0 -> 16.4; 256 rows 4.7
+// against 5.0.  Four rows leave too few workgroups (384 rows 7.1, 2112 16.6).
+template <typename T, int R, int N>
+__global__ __launch_bounds__(512) void add_rmsnorm_rows_kernel(
+    T* __restrict__ r, int64_t ldr, const T* __restrict__ x, int64_t ldx, const T* __restrict__ w,
+    T* __restrict__ out, int64_t ldo, int rows, int hidden, float eps, LoraUp lora) {
+  static_assert(R > 0 && R <= 16, "B of eight columns in registers");
+  __shared__ float s_red[N][512 / kWave];
+  const int row0 = blockIdx.x * N;
+  const bool live = (int)threadIdx.x * 8 < hidden;
+  const int idx = live ? threadIdx.x * 8 : hidden - 8;
+  uint4 b[8][R / 8], xw[N], rw[N];
+  LoraRow<R> y[N];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int k = 0; k < R / 8; ++k) b[i][k] = *lora_b_piece<T, R>(lora, lora.adapter, idx, i, k);
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const int64_t row = min(row0 + n, rows - 1);
+    xw[n] = *reinterpret_cast<const uint4*>(x + row * ldx + idx);
+    rw[n] = *reinterpret_cast<const uint4*>(r + row * ldr + idx);
+    load_y<T, R>(lora, row, lora.adapter, y[n]);
+  }
+  float wf[8];
+  load_row8<T>(w + idx, wf);
+  __builtin_amdgcn_sched_barrier(0);  // every load in flight
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    float v[8], xa[8];
+    load_row8<T>(reinterpret_cast<const T*>(&xw[n]), xa);
+    load_row8<T>(reinterpret_cast<const T*>(&rw[n]), v);
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float acc = 0.f;
+#pragma unroll
+      for (int k = 0; k < R / 8; ++k) acc = dot8<T>(y[n].v[k], b[i][k], acc);
+      v[i] = through<T>(v[i] + through<T>(xa[i] + acc * lora.scale));
+      ss = fmaf(v[i], v[i], ss);
+    }
+    store_row8<T>(reinterpret_cast<T*>(&rw[n]), v);
+    ss = wave_sum(live ? ss : 0.f);
+    if (lane == 0) s_red[n][wave] = ss;
+  }
+  __syncthreads();
+  const int nw = blockDim.x / kWave;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const int64_t row = row0 + n;
+    if (row >= rows) break;
+    float tot = 0.f;
+    for (int i = 0; i < nw; ++i) tot += s_red[n][i];
+    const float rstd = rsqrtf(tot / (float)hidden + eps);
+    float v[8];
+    load_row8<T>(reinterpret_cast<const T*>(&rw[n]), v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = v[i] * rstd * wf[i];
+    if (live) {
+      *reinterpret_cast<uint4*>(r + row * ldr + idx) = rw[n];
+      store_row8<T>(out + row * ldo + idx, v);
+    }
+  }
 }
 
 // One 8-column chunk per thread.  R > 0: lg / lu are the gate and up
@@ -809,6 +880,20 @@ static int launch_norm(bool add, int rank, void* r, int64_t ldr, const void* x, 
                        const int32_t* ids, int na, const SplitIn& xs, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
     // decode-sized rows: the single-chunk kernel (two memory round trips)
+    if (add && xs.splits == 0 && (rank == 8 || rank == 16) && lu.adapter >= 0 && rows >= kNormRowsMin &&
+        hidden <= 4096) {
+      const int threads = (hidden / 8 + kWave - 1) / kWave * kWave;
+      auto go = [&](auto rk) {
+        constexpr int R = decltype(rk)::value;
+        hipLaunchKernelGGL((add_rmsnorm_rows_kernel<T, R, kNormRows>), dim3((rows + kNormRows - 1) / kNormRows),
+                           dim3(threads), 0, s, (T*)r, ldr, (const T*)x, ldx, (const T*)w, (T*)out, ldo, rows, hidden,
+                           eps, lu);
+      };
+      if (rank == 8) go(std::integral_constant<int, 8>{});
+      else go(std::integral_constant<int, 16>{});
+      PL_LAUNCH_CHECK("add_rmsnorm_rows_kernel");
+      return ok();
+    }
     if (add && hidden <= kRowNormMaxHidden && xs.splits <= 4) {
       switch (xs.splits) {
         case 0: launch_row_norm_p<T, 0>(rank, r, ldr, x, ldx, w, out, ldo, rows, hidden, eps, lu, ids, na, xs, s); break;

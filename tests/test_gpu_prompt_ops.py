@@ -75,3 +75,27 @@ def test_qk_norm_rope_append(gpu_device, dtype, rank, rows, hq, hkv, norm):
     for got, want in zip(*results):
         _close(got, want, dtype)
     assert ((results[0][1] != 0) == (results[1][1] != 0)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rank", [8, 16])
+@pytest.mark.parametrize("rows,hidden", [(320, 8), (321, 520), (1027, 4096), (323, 4088)])
+@pytest.mark.parametrize("chunk8", [False, True])
+def test_add_rmsnorm_rows(gpu_device, dtype, rank, rows, hidden, chunk8):
+    """Rows sharing B in registers vs a row per workgroup."""
+    gen = torch.Generator().manual_seed(rows + hidden + rank)
+    n = 2
+    x = torch.randn((rows, hidden + n * rank), generator=gen).to(dtype).to(gpu_device)
+    res = torch.randn((rows, hidden), generator=gen).to(dtype).to(gpu_device)
+    w = (1 + 0.1 * torch.randn(hidden, generator=gen)).to(dtype).to(gpu_device)
+    B = (torch.randn((n, hidden, rank), generator=gen) * 0.1).to(dtype).to(gpu_device)
+    Bs = fused_ops.lora_b_chunk8(B) if chunk8 else B
+    ids = torch.ones(rows, dtype=torch.int32, device=gpu_device)
+    outs = []
+    for a in (1, -1):
+        r = res.clone()
+        m = fused_ops.LoraUp(x, hidden, Bs, 2.0, a)
+        outs.append((fused_ops.add_rmsnorm(r, x[:, :hidden], w, 1e-6, lora=m, adapter_ids=ids), r))
+    torch.cuda.synchronize()
+    for got, want in zip(*outs):
+        _close(got, want, dtype)
