@@ -26,6 +26,14 @@ struct TileArgs {
   int tokens, K, N, m_tiles, n_tiles, splits, vec_out;
 };
 
+// Where split s of `splits` (a power of two) begins, in 64-wide steps of K.
+// An even division: with steps >= splits every split has at least one step
+// (ceil(steps / splits) steps each would leave the last of 8 splits of 33
+// steps empty, and a workgroup loads its first step unasked).
+__host__ __device__ inline int split_begin(int steps, int splits, int s) {
+  return (int)(((unsigned)steps * (unsigned)s) / (unsigned)splits);
+}
+
 // 32-bit byte offsets reach every row of a token tile.
 bool wide_supports(int64_t ldx);
 

@@ -166,8 +166,10 @@ template <int N> __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0xF70);
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0xffffffffu, 0x00027000);
+// A buffer of `bytes` from p on; loads past it read 0.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (uint32_t)min(bytes, (int64_t)0xffffffff),
+                                           0x00027000);
 }
 
 template <typename T, int MF, int NF, int S>
@@ -201,18 +203,19 @@ __device__ __forceinline__ void tile_gemm(const TileArgs& g) {
   const int mt = id % g.m_tiles, nt = (id / g.m_tiles) % g.n_tiles, split = id / (g.m_tiles * g.n_tiles);
   const int t0 = mt * BM;
   const int all_steps = g.K / 64;
-  const int per_split = (all_steps + g.splits - 1) / g.splits;
-  const int step0 = min(all_steps, split * per_split);
-  const int steps = min(all_steps, step0 + per_split) - step0;
+  const int step0 = split_begin(all_steps, g.splits, split);
+  const int steps = split_begin(all_steps, g.splits, split + 1) - step0;  // >= 1
   const int ksteps = g.K / 32;
   const int n_blocks = (g.N + 15) / 16;
   const int nb0 = nt * (8 * NF) + wave * NF;
 
-  // buffer descriptors: the wave's weight blocks and the tile's x rows
-  // (clamped, so neither reads past its tensor), offsets in scalar registers
+  // buffer descriptors: the wave's weight blocks and the tile's x rows, each
+  // to its tensor's end (blocks, rows and steps past the last are clamped to
+  // it), offsets in scalar registers
   const int nbc = min(nb0, n_blocks - 1);
-  const auto wr = make_rsrc((const char*)g.W + ((int64_t)nbc * ksteps + 2 * step0) * kBlockBytes);
-  const auto xr = make_rsrc((const char*)g.x + (int64_t)t0 * g.ldx * 2 + step0 * 128);
+  const int64_t w_at = ((int64_t)nbc * ksteps + 2 * step0) * kBlockBytes, x_at = (int64_t)t0 * g.ldx * 2 + step0 * 128;
+  const auto wr = make_rsrc((const char*)g.W + w_at, (int64_t)n_blocks * ksteps * kBlockBytes - w_at);
+  const auto xr = make_rsrc((const char*)g.x + x_at, ((int64_t)(g.tokens - 1) * g.ldx + g.K) * 2 - x_at);
   int wso[NF];
 #pragma unroll
   for (int n = 0; n < NF; ++n) wso[n] = uniform((min(nb0 + n, n_blocks - 1) - nbc) * ksteps * kBlockBytes);
@@ -250,7 +253,7 @@ __device__ __forceinline__ void tile_gemm(const TileArgs& g) {
     for (int n = 0; n < NF; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   u32x4 w[S][2][NF];
-  const int last = max(steps - 1, 0);
+  const int last = steps - 1;
 #pragma unroll
   for (int p = 0; p < S - 1; ++p) {
     load_x(min(p, last), buf(p));
@@ -511,6 +514,15 @@ extern "C" size_t pl_linear_shuffled_wide_workspace_size(int num_tokens, int in_
   if (num_tokens <= kStripMaxTokens || in_features <= 0 || in_features % 64 || out_features <= 0) return 0;
   const Choice c = choose(num_tokens, out_features, in_features, true);
   return c.splits > 1 ? (size_t)c.splits * num_tokens * split_ld(out_features) * sizeof(float) : 0;
+}
+
+extern "C" int pl_linear_shuffled_wide_splits(int num_tokens, int in_features, int out_features,
+                                              int32_t* step_begin_h) {
+  if (num_tokens <= kStripMaxTokens || in_features <= 0 || in_features % 64 || out_features <= 0) return 1;
+  const int splits = choose(num_tokens, out_features, in_features, true).splits;
+  for (int s = 0; s <= splits && step_begin_h != nullptr; ++s)
+    step_begin_h[s] = split_begin(in_features / 64, splits, s);
+  return splits;
 }
 
 extern "C" int pl_linear_shuffled_wide(const void* x, int64_t ldx, int num_tokens, int in_features,

@@ -44,6 +44,15 @@ def test_linear_wide_vs_oracle(gpu_device, dtype, tokens, n, k):
     assert (err <= 2e-3 + REL[dtype] * np.abs(want)).all(), f"max err {err.max():.3e}"
 
 
+# K steps that their splits do not divide evenly (33, 42, 65 by 8, 19 by 4, 33 by 2)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,n,k,splits", [(48, 1000, 2112, 8), (64, 4096, 2688, 8), (65, 1000, 4160, 8),
+                                               (49, 37, 1216, 4), (40, 8208, 2112, 2)])
+def test_uneven_splits(gpu_device, dtype, tokens, n, k, splits):
+    assert _lib.load().pl_linear_shuffled_wide_splits(tokens, k, n, None) == splits
+    test_linear_wide_vs_oracle(gpu_device, dtype, tokens, n, k)
+
+
 def test_strided_x_without_workspace(gpu_device):
     """x as a column slice of a wider buffer; no workspace: the same product
     with its K sums in one piece."""
