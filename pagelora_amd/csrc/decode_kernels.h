@@ -381,15 +381,20 @@ template <> __device__ __forceinline__ f32x4 mfma_16x16x16<f16_t>(uint2 a, uint2
 // A probability pair as two planes of T: the value cut to T, and what the cut
 // left (bf16: 16 bits of the mantissa, fp16: 22).  Both planes stay above zero
 // (by T's least useful value), so an infinite V gives the infinity that the
-// product with the whole probability gives, not 0 * inf.
+// product with the whole probability gives, not 0 * inf.  fp16 holds the
+// probabilities times 2^14, which puts that least value at 2^-38 of the
+// maximum: 32768 tokens far below it then add 1e-7 of one's V, not 4e-3 as
+// without the factor.
 template <typename T> struct PlanePair;
 template <> struct PlanePair<bf16_t> {
+  static constexpr float kScale = 1.f;
   static constexpr float kTiny = 1.17549435e-38f;
   static __device__ __forceinline__ uint32_t cut(float a, float b) {
     return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
   }
 };
 template <> struct PlanePair<f16_t> {
+  static constexpr float kScale = 16384.f;
   static constexpr float kTiny = 5.9604645e-8f;
   static __device__ __forceinline__ uint32_t cut(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
@@ -425,7 +430,7 @@ struct DecodeWaveMatrix {
 
   uint32_t qb[NS][W];  // B operand: head lane % 16, dims 32 j + 8 (lane / 16) ..
   float mo, lo;        // head lane % 16: running max (all lane rows), sum of this lane row's tokens
-  f32x4 acc[8];        // acc[d][i]: dim 32 (lane / 16) + 8 i + d of head lane % 16
+  f32x4 acc[8];        // acc[d][i]: dim 32 (lane / 16) + 8 i + d of head lane % 16, times PlanePair's scale
 
   __device__ void init() {
     mo = -INFINITY;
@@ -482,6 +487,7 @@ struct DecodeWaveMatrix {
       for (int e = 0; e < 2; ++e) {
         p[e] = fast_exp2(sc[2 * k + e] - m_use);
         lo += p[e];
+        p[e] *= PP::kScale;
         p[e] = fmaxf(p[e], PP::kTiny) + (p[e] != p[e] ? p[e] : 0.f);  // (a NaN stays one)
       }
       hi[k] = PP::cut(p[0], p[1]);
@@ -1339,7 +1345,7 @@ __global__ __launch_bounds__(kWave * waves_per_wg<FUSED>()) void decode_kernel(
     const int g = lane % 16;
     if (g >= G) return;
     const int hq = h * G + g;
-    const float inv = st.lo > 0.f ? 1.f / st.lo : 0.f;
+    const float inv = st.lo > 0.f ? 1.f / (st.lo * PlanePair<T>::kScale) : 0.f;
     const int64_t slot_row = (int64_t)(flags >> 2) * num_qo_heads + hq;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

@@ -1,0 +1,62 @@
+"""The probability planes of the decode wave for groups of 4 heads and more, vs
+the float64 oracle: one row of few items, scores and V chosen so that what the
+planes drop or add shows in the result."""
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import paged_decode as opd
+from tests.gpu_cases import ragged_case
+from tests.test_gpu_decode_matrix import _run
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.bfloat16, torch.float16]
+REL = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}
+
+
+def _one_row(scores, v, group, dtype, device):
+    """One row of ``group`` heads that all score token t ``scores[t]`` (in
+    powers of two) and read V rows ``v`` [tokens, 128]."""
+    n = len(scores)
+    case = ragged_case(lens=[n], hq=group, hkv=1, head_dim=128, page_size=16, dtype=dtype, device="cpu", seed=1)
+    # q = 8 in dim 0, K = the score there: q . K / sqrt(128) * log2(e) = score
+    q, cache = torch.zeros_like(case["q"]), torch.zeros_like(case["cache"])
+    q[:, :, 0] = 8.0
+    pages = case["indices"].long()
+    k = torch.zeros((len(pages) * 16, 128))
+    k[:n, 0] = torch.as_tensor(scores, dtype=torch.float32) * (math.sqrt(128) / 8.0 / math.log2(math.e))
+    vv = torch.zeros((len(pages) * 16, 128))
+    vv[:n] = torch.as_tensor(v, dtype=torch.float32)
+    cache[pages, 0, :, 0] = k.reshape(-1, 16, 128).to(dtype)
+    cache[pages, 1, :, 0] = vv.reshape(-1, 16, 128).to(dtype)
+    case["q_host"], case["cache_host"] = q, cache
+    case["q"], case["cache"] = q.to(device), cache.to(device)
+    return case
+
+
+def _want(case):
+    return opd.paged_decode(case["q_host"].float().numpy(), case["cache_host"].float().numpy(),
+                            case["indptr"].numpy(), case["indices"].numpy(), case["last"].numpy())[0]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("group", [4, 7])
+@pytest.mark.parametrize("n", [2048, 16384])
+@pytest.mark.parametrize("below", [30.0, 60.0])
+def test_tokens_far_below_the_maximum_add_nothing(gpu_device, dtype, group, n, below):
+    """One token (an attention sink with a small V) far above n others with V =
+    1, in one item: the others weigh n 2^-below.  Bar: one rounding of the
+    result, and 2^-36 of V for every token."""
+    scores = np.zeros(n)
+    scores[0] = below
+    v = np.ones((n, 128))
+    v[0] = 0.05
+    case = _one_row(scores, v, group, dtype, gpu_device)
+    got = _run(case, group, 1, 16, gpu_device, target_waves=1)
+    want = _want(case)
+    err = np.abs(got - want)
+    assert (err <= REL[dtype] * np.abs(want) + n * 2.0**-36).all(), f"max err {err.max():.3e}"
