@@ -379,12 +379,12 @@ template <> __device__ __forceinline__ f32x4 mfma_16x16x16<f16_t>(uint2 a, uint2
 }
 
 // A probability pair as two planes of T: the value cut to T, and what the cut
-// left (bf16: 16 bits of the mantissa, fp16: 22).  Both planes stay above zero
-// (by T's least useful value), so an infinite V gives the infinity that the
-// product with the whole probability gives, not 0 * inf.  fp16 holds the
-// probabilities times 2^14, which puts that least value at 2^-38 of the
-// maximum: 32768 tokens far below it then add 1e-7 of one's V, not 4e-3 as
-// without the factor.
+// left (bf16: 16 bits of the mantissa, fp16: 22).  Where the probability is
+// above 0 both planes are too (by T's least useful value), so an infinite V
+// gives what its product with the whole probability gives: an infinity, and
+// NaN where the probability is 0.  fp16 holds the probabilities times 2^14,
+// which puts that least value at 2^-38 of the maximum: 32768 tokens far below
+// it then add 1e-7 of one's V, not 4e-3 as without the factor.
 template <typename T> struct PlanePair;
 template <> struct PlanePair<bf16_t> {
   static constexpr float kScale = 1.f;
@@ -482,17 +482,18 @@ struct DecodeWaveMatrix {
     uint32_t hi[2], low[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      float p[2], h[2];
+      float p[2], h[2], tiny[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         p[e] = fast_exp2(sc[2 * k + e] - m_use);
         lo += p[e];
+        tiny[e] = p[e] > 0.f ? PP::kTiny : 0.f;
         p[e] *= PP::kScale;
-        p[e] = fmaxf(p[e], PP::kTiny) + (p[e] != p[e] ? p[e] : 0.f);  // (a NaN stays one)
+        p[e] = p[e] < tiny[e] ? tiny[e] : p[e];  // (a NaN stays one)
       }
       hi[k] = PP::cut(p[0], p[1]);
       unpack2<T>(hi[k], h[0], h[1]);
-      low[k] = pack2_hw<T>(fmaxf(p[0] - h[0], PP::kTiny), fmaxf(p[1] - h[1], PP::kTiny));
+      low[k] = pack2_hw<T>(fmaxf(p[0] - h[0], tiny[0]), fmaxf(p[1] - h[1], tiny[1]));
     }
     const uint2 bh = make_uint2(hi[0], hi[1]), bl = make_uint2(low[0], low[1]);
 #pragma unroll

@@ -60,3 +60,25 @@ def test_tokens_far_below_the_maximum_add_nothing(gpu_device, dtype, group, n, b
     want = _want(case)
     err = np.abs(got - want)
     assert (err <= REL[dtype] * np.abs(want) + n * 2.0**-36).all(), f"max err {err.max():.3e}"
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("group", [2, 4, 7])
+@pytest.mark.parametrize("first", [True, False])
+def test_infinite_v_at_a_probability_of_zero_is_nan(gpu_device, dtype, group, first):
+    """A token 400 powers of two below the maximum has probability 0 in fp32:
+    an infinite V there gives 0 * inf = NaN in its dim for every group size
+    (2 heads: the vector wave), whichever of the two tokens comes first, and
+    nothing in the other dims."""
+    n = 100
+    scores = np.zeros(n)
+    scores[0 if first else 90] = 400.0
+    v = np.random.default_rng(2).standard_normal((n, 128))
+    v[37, 9] = np.inf
+    case = _one_row(scores, v, group, dtype, gpu_device)
+    got = _run(case, group, 1, 16, gpu_device, target_waves=1)
+    case["cache_host"][case["cache_host"].isinf()] = 0.0
+    want = _want(case)
+    assert np.isnan(got[:, :, 9]).all()
+    rest = np.arange(128) != 9
+    assert (np.abs(got - want)[:, :, rest] <= REL[dtype] * np.abs(want[:, :, rest]) + 1e-6).all()
