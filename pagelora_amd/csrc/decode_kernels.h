@@ -378,22 +378,28 @@ template <> __device__ __forceinline__ f32x4 mfma_16x16x16<f16_t>(uint2 a, uint2
                                                0);
 }
 
-// A probability pair as two planes of T: the value cut to T, and what the cut
-// left (bf16: 16 bits of the mantissa, fp16: 22).  Where the probability is
-// above 0 both planes are too (by T's least useful value), so an infinite V
-// gives what its product with the whole probability gives: an infinity, and
-// NaN where the probability is 0.  fp16 holds the probabilities times 2^14,
-// which puts that least value at 2^-38 of the maximum: 32768 tokens far below
-// it then add 1e-7 of one's V, not 4e-3 as without the factor.
-template <typename T> struct PlanePair;
-template <> struct PlanePair<bf16_t> {
+// Probabilities as three planes of T: the value cut to T, what the cut left cut
+// to T, and the rest, which T holds whole.  So P . V has the fp32 value's 24
+// bits (two planes hold 16 in bf16 and 22 in fp16: three terms that cancel to
+// 2^-12 of themselves came out 4.3e-2 off in bf16, against 2.3e-3).  Where the
+// probability is above 0 every plane is too (by T's least useful value), so an
+// infinite V gives what its product with the whole probability gives: an
+// infinity, and NaN where the probability is 0.  fp16 holds the probabilities
+// times 2^14, which puts that least value at 2^-38 of the maximum: 32768
+// tokens far below it then add 4e-7 of one's V, not 4e-3 as without the factor.
+// The third plane's cutting and MFMAs cost 1 to 3 %, back to back in a graph:
+// 1 x 2048 9.2 -> 9.35 us, 64 x 2048 (GQA 4) 90.9 -> 92.0, 64 x 8192 344.8 ->
+// 348.0, 23 ragged rows of 7 heads 28.8 -> 29.2 (the planes' order over the
+// tiles, and two of them in one 16x16x32 tile, made no difference).
+template <typename T> struct ProbPlanes;
+template <> struct ProbPlanes<bf16_t> {
   static constexpr float kScale = 1.f;
   static constexpr float kTiny = 1.17549435e-38f;
   static __device__ __forceinline__ uint32_t cut(float a, float b) {
     return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
   }
 };
-template <> struct PlanePair<f16_t> {
+template <> struct ProbPlanes<f16_t> {
   static constexpr float kScale = 16384.f;
   static constexpr float kTiny = 5.9604645e-8f;
   static __device__ __forceinline__ uint32_t cut(float a, float b) {
@@ -425,12 +431,13 @@ struct DecodeWaveMatrix {
   static constexpr int NS = kBlockTokens / TPI;
   static constexpr int W = 4;
   static constexpr bool kMfmaScores = true;
+  static constexpr int kPlanes = 3;
   using L8 = Lane8<T>;
   static_assert(NS == 4, "four token rows per lane: one k group of the 16x16x16 tile");
 
   uint32_t qb[NS][W];  // B operand: head lane % 16, dims 32 j + 8 (lane / 16) ..
   float mo, lo;        // head lane % 16: running max (all lane rows), sum of this lane row's tokens
-  f32x4 acc[8];        // acc[d][i]: dim 32 (lane / 16) + 8 i + d of head lane % 16, times PlanePair's scale
+  f32x4 acc[8];        // acc[d][i]: dim 32 (lane / 16) + 8 i + d of head lane % 16, times ProbPlanes's scale
 
   __device__ void init() {
     mo = -INFINITY;
@@ -478,11 +485,11 @@ struct DecodeWaveMatrix {
         for (int i = 0; i < 4; ++i) acc[d][i] *= alpha;
     }
     const float m_use = mo == -INFINITY ? 0.f : mo;
-    using PP = PlanePair<T>;
-    uint32_t hi[2], low[2];
+    using PP = ProbPlanes<T>;
+    uint32_t pw[kPlanes][2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      float p[2], h[2], tiny[2];
+      float p[2], tiny[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         p[e] = fast_exp2(sc[2 * k + e] - m_use);
@@ -491,18 +498,22 @@ struct DecodeWaveMatrix {
         p[e] *= PP::kScale;
         p[e] = p[e] < tiny[e] ? tiny[e] : p[e];  // (a NaN stays one)
       }
-      hi[k] = PP::cut(p[0], p[1]);
-      unpack2<T>(hi[k], h[0], h[1]);
-      low[k] = pack2_hw<T>(fmaxf(p[0] - h[0], tiny[0]), fmaxf(p[1] - h[1], tiny[1]));
+#pragma unroll
+      for (int n = 0; n < kPlanes; ++n) {
+        pw[n][k] = PP::cut(p[0], p[1]);
+        float h[2];
+        unpack2<T>(pw[n][k], h[0], h[1]);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) p[e] = fmaxf(p[e] - h[e], tiny[e]);
+      }
     }
-    const uint2 bh = make_uint2(hi[0], hi[1]), bl = make_uint2(low[0], low[1]);
 #pragma unroll
     for (int d = 0; d < 8; ++d) {
       const uint32_t sel = d % 2 ? 0x07060302u : 0x05040100u;
       const uint2 a = make_uint2(__builtin_amdgcn_perm(vw[1][d / 2], vw[0][d / 2], sel),
                                  __builtin_amdgcn_perm(vw[3][d / 2], vw[2][d / 2], sel));
-      acc[d] = mfma_16x16x16<T>(a, bh, acc[d]);
-      acc[d] = mfma_16x16x16<T>(a, bl, acc[d]);
+#pragma unroll
+      for (int n = 0; n < kPlanes; ++n) acc[d] = mfma_16x16x16<T>(a, make_uint2(pw[n][0], pw[n][1]), acc[d]);
     }
   }
 
@@ -1346,7 +1357,7 @@ __global__ __launch_bounds__(kWave * waves_per_wg<FUSED>()) void decode_kernel(
     const int g = lane % 16;
     if (g >= G) return;
     const int hq = h * G + g;
-    const float inv = st.lo > 0.f ? 1.f / (st.lo * PlanePair<T>::kScale) : 0.f;
+    const float inv = st.lo > 0.f ? 1.f / (st.lo * ProbPlanes<T>::kScale) : 0.f;
     const int64_t slot_row = (int64_t)(flags >> 2) * num_qo_heads + hq;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

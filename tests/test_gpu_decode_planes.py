@@ -82,3 +82,38 @@ def test_infinite_v_at_a_probability_of_zero_is_nan(gpu_device, dtype, group, fi
     assert np.isnan(got[:, :, 9]).all()
     rest = np.arange(128) != 9
     assert (np.abs(got - want)[:, :, rest] <= REL[dtype] * np.abs(want[:, :, rest]) + 1e-6).all()
+
+
+def _cancelling_error(group, dtype, device, seed):
+    """The relative error of a row whose three terms nearly cancel."""
+    rng = np.random.default_rng(seed)
+    scores = np.array([0.0, -rng.uniform(0.1, 0.9), -rng.uniform(1.1, 1.9)])
+    v = np.zeros((3, 128))
+    case = _one_row(scores, v, group, dtype, device)
+    page = int(case["indices"][0])
+    k0 = case["cache_host"][page, 0, :3, 0, 0].double().numpy()
+    p = np.exp((k0 - k0.max()) * 8.0 / math.sqrt(128))
+    cut = lambda x: torch.as_tensor(x, dtype=torch.float64).to(dtype).double().numpy()  # noqa: E731
+    v[1] = cut(rng.uniform(1, 2, 128))
+    v[0] = cut(-p[1] * v[1] / p[0])
+    left = p[0] * v[0] + p[1] * v[1]
+    v[2] = cut(-(left - np.sign(left) * 2.0**-12) / p[2])  # takes the rest down to about 2^-12 of the terms
+    for key in ("cache", "cache_host"):
+        case[key][page, 1, :3, 0] = torch.as_tensor(v).to(dtype).to(case[key].device)
+    got, want = _run(case, group, 1, 16, device, target_waves=1), _want(case)
+    return np.linalg.norm(got - want) / np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("group", [4, 7])
+def test_probabilities_keep_their_32_bits(gpu_device, dtype, group):
+    """Terms that cancel down to 2^-12 of themselves: a probability of 16 bits
+    leaves an error of up to 2^-5 of the result, one of 22 bits 2^-11.  The
+    vector wave (2 heads; fp32 probabilities, and the same scores, of which
+    only one dim is not zero) is the measure; beyond its error 2^-13 for the
+    order of the sums (2^-24 of the terms, twice)."""
+    errs = [(_cancelling_error(group, dtype, gpu_device, s), _cancelling_error(2, dtype, gpu_device, s))
+            for s in range(8)]
+    print(f"[planes] {dtype} group {group}: worst " + ", vector wave ".join(f"{max(e):.2e}" for e in zip(*errs)),
+          flush=True)
+    assert all(a <= b + 2.0**-13 for a, b in errs), errs
