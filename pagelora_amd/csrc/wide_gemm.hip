@@ -536,10 +536,17 @@ extern "C" int pl_linear_shuffled_wide(const void* x, int64_t ldx, int num_token
   if (ldx < in_features || ldx % 8 || (uintptr_t)x % 16 || (uintptr_t)shuffled % 16)
     return fail(PL_ERR_INVALID, "x rows and the shuffled weight must be 16-byte aligned");
   if (ldo < out_features) return fail(PL_ERR_INVALID, "ldo < out_features");
-  if (!wide_supports(ldx)) return fail(PL_ERR_UNSUPPORTED, "ldx %lld too large", (long long)ldx);
   if ((uintptr_t)workspace % 16) return fail(PL_ERR_INVALID, "workspace must be 16-byte aligned");
   if (dtype != PL_DTYPE_BF16 && dtype != PL_DTYPE_F16)
     return fail(PL_ERR_UNSUPPORTED, "pl_linear_shuffled_wide dtype must be F16 or BF16 (got %d)", dtype);
+  if (!wide_supports(ldx)) {  // rows too far apart for these kernels' offsets: 64 of them at a time
+    for (int t = 0; t < num_tokens; t += PL_LINEAR_MAX_TOKENS)
+      if (const int st = pl_linear_shuffled((const char*)x + (int64_t)t * ldx * 2, ldx,
+                                            std::min(num_tokens - t, PL_LINEAR_MAX_TOKENS), in_features, shuffled,
+                                            out_features, bias, (char*)out + (int64_t)t * ldo * 2, ldo, dtype, stream))
+        return st;
+    return ok();
+  }
   const int st = wide_linear(x, ldx, num_tokens, in_features, shuffled, out_features, bias, out, ldo, workspace,
                              workspace_bytes, dtype, (hipStream_t)stream);
   return st ? st : ok();

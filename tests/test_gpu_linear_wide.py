@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from pagelora_amd import _lib
-from pagelora_amd.linear import ShuffledWeight, linear_shuffled_wide
+from pagelora_amd.linear import ShuffledWeight, linear_shuffled, linear_shuffled_wide
 
 pytestmark = pytest.mark.gpu
 
@@ -71,4 +71,21 @@ def test_strided_x_without_workspace(gpu_device):
     want = x.double().cpu().numpy() @ w.double().cpu().numpy().T
     for got in (out, split):
         err = np.abs(got.float().cpu().numpy() - want)
+        assert (err <= 2e-3 + 2.0**-8 * np.abs(want)).all(), f"max err {err.max():.3e}"
+
+
+@pytest.mark.parametrize("tokens", [17, 64, 70])
+def test_rows_far_apart(gpu_device, tokens):
+    """A row stride of 2^22 elements, past the tile kernels' 32-bit offsets:
+    the same product, by the 16-token kernel."""
+    k, n = 96, 40
+    g = torch.Generator(device=gpu_device).manual_seed(tokens)
+    x = torch.empty(((tokens - 1) << 22) + k, dtype=torch.bfloat16, device=gpu_device).as_strided(
+        (tokens, k), (1 << 22, 1))
+    x.copy_(torch.randn((tokens, k), generator=g, device=gpu_device))
+    w = (torch.randn((n, k), generator=g, device=gpu_device) * k ** -0.5).to(torch.bfloat16)
+    sw = ShuffledWeight(w)
+    want = x.double().cpu().numpy() @ w.double().cpu().numpy().T
+    for call in (linear_shuffled_wide, linear_shuffled)[: 2 if tokens <= 64 else 1]:
+        err = np.abs(call(x, sw).float().cpu().numpy() - want)
         assert (err <= 2e-3 + 2.0**-8 * np.abs(want)).all(), f"max err {err.max():.3e}"
