@@ -356,11 +356,19 @@ class DecoderWeights:
         return self._lm_head if self._lm_head is not None else self.lm_head_shuffled.unshuffle()
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
-        """x . lm_head^T: the shuffled GEMM where that copy was made, else the
-        library GEMM on the row-major weight."""
-        if self.lm_head_shuffled is not None:
-            return linear_shuffled_wide(x, self.lm_head_shuffled)
-        return F.linear(x, self._lm_head)
+        """x . lm_head^T: the shuffled GEMM where that copy was made.  Past the
+        decode GEMM's rows (16, or 64 when no row-major copy is kept) an x that
+        it does not take (column strides, other shapes, unaligned rows,
+        gradients) goes through the library GEMM on the row-major weight."""
+        sw = self.lm_head_shuffled
+        if sw is not None:
+            limit = _lib.PL_LINEAR_MAX_TOKENS if self._lm_head is None else DECODE_GEMM_MAX_TOKENS
+            if x.shape[0] <= limit or (x.dim() == 2 and x.shape[1] == sw.in_features and x.stride(1) == 1
+                                       and x.stride(0) >= x.shape[1] and x.stride(0) % 8 == 0
+                                       and x.data_ptr() % 16 == 0 and x.dtype == sw.dtype and x.is_cuda
+                                       and not (x.requires_grad and torch.is_grad_enabled())):
+                return linear_shuffled_wide(x, sw)
+        return F.linear(x, self.lm_head)
 
     @classmethod
     def from_tensors(cls, cfg: DecoderConfig, *, embed: torch.Tensor, final_norm: torch.Tensor,
