@@ -51,21 +51,31 @@ def reserve_workspace(device: torch.device | str, nbytes: int) -> None:
 
 
 _DELTA_WS: dict[int, torch.Tensor] = {}
+_UNSIZED = "LoRA workspace must be sized before graph capture (call reserve_delta_workspace)"
 
 
 def _delta_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """Per-device workspace of pl_lora_delta(_groups): zero-filled when
     allocated (its ticket area must start at zero; every call leaves it so)
     and used by no other entry point; grown on demand, never inside a
-    captured graph."""
+    captured graph.  There a buffer below ``nbytes`` is returned as it is: the
+    call then takes the path that needs less, or refuses."""
     key = device.index if device.index is not None else torch.cuda.current_device()
     ws = _DELTA_WS.get(key)
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
-            raise RuntimeError("LoRA workspace must be sized before graph capture (call reserve_delta_workspace)")
+            if ws is None:
+                raise RuntimeError(_UNSIZED)
+            return ws
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _DELTA_WS[key] = ws
     return ws
+
+
+def _check_delta(status: int, what: str) -> None:
+    if status == _lib.PL_ERR_WORKSPACE:  # only a capture is given less than it asked for
+        raise RuntimeError(_UNSIZED)
+    _lib.check(status, what)
 
 
 def reserve_delta_workspace(device: torch.device | str, nbytes: int) -> None:
@@ -141,7 +151,7 @@ def lora_delta_(
         adapter_ids.data_ptr(), n_adapters, _lib.dtype_code(x.dtype), _lib.dtype_code(out_dtype),
         ws.data_ptr(), ws.numel(), _lib.stream_handle(x.device),
     )
-    _lib.check(status, "pl_lora_delta")
+    _check_delta(status, "pl_lora_delta")
 
 
 def lora_delta_groups_(
@@ -183,7 +193,7 @@ def lora_delta_groups_(
         descs, len(groups), T, adapter_ids.data_ptr(), n_adapters, _lib.dtype_code(x0.dtype),
         _lib.dtype_code(out_dtype), ws.data_ptr(), ws.numel(), _lib.stream_handle(x0.device),
     )
-    _lib.check(status, "pl_lora_delta_groups")
+    _check_delta(status, "pl_lora_delta_groups")
 
 
 def lora_linear(

@@ -88,3 +88,49 @@ def test_groups_in_sequence_where_one_reads_anothers_output(gpu_device):
     torch.cuda.synchronize()
     assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
     assert results[0][1].abs().sum() > 0
+
+
+def test_capture_with_the_general_path_s_workspace(gpu_device, monkeypatch):
+    """A capture of many tokens with a workspace that holds the general path's
+    partials but not the tiles' buffers takes the general path; one that holds
+    neither is refused before anything is recorded."""
+    from pagelora_amd import _lib, lora
+
+    gen = torch.Generator().manual_seed(5)
+    T, spec = 4096, [(64, [(16, 16)])] * 4
+    groups, host = _case(T, 2, spec, torch.bfloat16, torch.bfloat16, gen, gpu_device)
+    ids = torch.randint(-1, 2, (T,), generator=gen, dtype=torch.int32).to(gpu_device)
+    descs = (_lib.LoraGroup * len(groups))()
+    keep = [lora._module_structs(mods, x)[0] for x, mods in groups]
+
+    def need():
+        for d, (x, mods), arr in zip(descs, groups, keep):
+            d.x, d.ldx, d.in_features, d.num_modules, d.modules = x.data_ptr(), x.stride(0), x.shape[1], len(mods), arr
+        return _lib.load().pl_lora_delta_workspace_size(descs, len(groups), T, 2)
+
+    tiled = need()
+    for arr in keep:
+        arr[0].out += 2  # an unaligned output: the general path's need (sizes only, nothing is read)
+    general = need()
+    assert general < tiled
+    for size in (general, general - 256):
+        monkeypatch.setitem(lora._DELTA_WS, gpu_device.index, torch.zeros(size, dtype=torch.uint8, device=gpu_device))
+        graph = torch.cuda.CUDAGraph()
+        refused = False
+        with torch.cuda.graph(graph):
+            try:
+                lora_delta_groups_(groups, ids)
+            except RuntimeError as e:
+                refused = "sized before graph capture" in str(e)
+        assert refused == (size < general)
+        if refused:
+            continue
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, A, B, base, got in host:
+            want = base
+            if x is not None:
+                want = base + ol.multi_adapter_delta(x.float().numpy(), ids.tolist(), A.float().numpy(),
+                                                     B.float().numpy(), 2.0, intermediate="bf16")
+            err = np.abs(got.float().cpu().numpy() - want)
+            assert (err <= 2e-3 + 2.0**-8 * np.abs(want)).all(), f"max err {err.max():.3e}"
