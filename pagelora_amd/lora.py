@@ -51,6 +51,7 @@ def reserve_workspace(device: torch.device | str, nbytes: int) -> None:
 
 
 _DELTA_WS: dict[int, torch.Tensor] = {}
+_OUTGROWN_WS: list[torch.Tensor] = []
 _UNSIZED = "LoRA workspace must be sized before graph capture (call reserve_delta_workspace)"
 
 
@@ -59,7 +60,10 @@ def _delta_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     allocated (its ticket area must start at zero; every call leaves it so)
     and used by no other entry point; grown on demand, never inside a
     captured graph.  There a buffer below ``nbytes`` is returned as it is: the
-    call then takes the path that needs less, or refuses."""
+    call then takes the path that needs less, or refuses.  A graph captured
+    before a growth replays into the buffer of its time, so outgrown buffers
+    are kept; each growth at least doubles, so all of them are smaller than
+    the one in use."""
     key = device.index if device.index is not None else torch.cuda.current_device()
     ws = _DELTA_WS.get(key)
     if ws is None or ws.numel() < nbytes:
@@ -67,6 +71,9 @@ def _delta_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
             if ws is None:
                 raise RuntimeError(_UNSIZED)
             return ws
+        if ws is not None:
+            _OUTGROWN_WS.append(ws)
+            nbytes = max(nbytes, 2 * ws.numel())
         ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _DELTA_WS[key] = ws
     return ws
