@@ -578,10 +578,18 @@ class PagedDecodeAttention:
         ``qo_len`` positions of its paged sequence; with ``causal`` query j
         sees kv positions ``<= kv_len - qo_len + j``.  The work list is built
         on the host (the tables are read there, as FlashInfer's prefill plan
-        does), then tables and work list are uploaded on the current stream,
-        without waiting for it (five copies that each did held the GPU idle
-        for 260 us of a 77-token prefill's plan).
+        does), then tables and work list are uploaded.  The upload is done
+        when this returns: a run may then be captured, on any stream.
         """
+        self._plan_prefill(qo_indptr, paged_kv_indptr, paged_kv_indices, paged_kv_last_page_len, causal, q_data_type,
+                           kv_data_type, wait=True)
+
+    def _plan_prefill(self, qo_indptr, paged_kv_indptr, paged_kv_indices, paged_kv_last_page_len, causal=True,
+                      q_data_type=None, kv_data_type=None, *, wait: bool) -> None:
+        """:meth:`plan_prefill`; with ``wait`` False the upload is only enqueued
+        on the current stream, for a caller that runs the plan next in the same
+        stream's order (waiting for the five tables in turn held the GPU idle
+        for 260 us of a 77-token prefill)."""
 
         tables = (qo_indptr, paged_kv_indptr, paged_kv_indices, paged_kv_last_page_len)
         if any(t.dim() != 1 for t in tables):
@@ -617,6 +625,9 @@ class PagedDecodeAttention:
         dev = _upload_int32((items_h, qo_h, kv_h, ind_h, last_h), self.device)
         items_d, *tables_d = dev
         stream = torch.cuda.current_stream(self.device)
+        ready = stream.record_event()
+        if wait:
+            ready.synchronize()
         self._prefill_plan = {
             "batch": batch,
             "tokens": int(qo_h[-1]) if batch else 0,
@@ -627,9 +638,9 @@ class PagedDecodeAttention:
             "causal": bool(causal),
             "max_page": max_page,
             "tables": (*tables_d, items_d),
-            # the upload is asynchronous: a run on another stream waits for it
             "stream": stream,
-            "ready": stream.record_event(),
+            # of an upload not waited for: a run on another stream waits for it
+            "ready": None if wait else ready,
             "q_data_type": q_data_type,
             "kv_data_type": kv_data_type,
         }
@@ -678,8 +689,8 @@ class PagedDecodeAttention:
         qo_d, kv_d, ind_d, last_d, items_d = plan["tables"]
         stream = torch.cuda.current_stream(q.device)
         if stream != plan["stream"] and not torch.cuda.is_current_stream_capturing():
-            # (a capture begins after a device synchronization, past the upload)
-            stream.wait_event(plan["ready"])
+            if plan["ready"] is not None:
+                stream.wait_event(plan["ready"])
             qo_d.record_stream(stream)  # one allocation holds every table
         if plan["split"]:
             # per call, from torch's allocator: calls on other streams share nothing

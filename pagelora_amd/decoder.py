@@ -35,6 +35,7 @@ prefill attention kernel.
 """
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass
 
 import torch
@@ -846,7 +847,12 @@ def prefill(weights: DecoderWeights, pool: PagedKVPool, request: Request, tokens
         T = tok.numel()
         ctx_len = start + c0 + T
         n_pages = -(-ctx_len // ps)
-        backend.plan_prefill(
+        # the runs follow in this stream's order, so the plan's upload need not
+        # be waited for (a backend's own plan_prefill is left as it is)
+        plan = backend.plan_prefill
+        if getattr(plan, "__func__", None) is PagedDecodeAttention.plan_prefill:
+            plan = functools.partial(backend._plan_prefill, wait=False)
+        plan(
             qo_indptr=torch.tensor([0, T], dtype=torch.int32),
             paged_kv_indptr=torch.tensor([0, n_pages], dtype=torch.int32),
             paged_kv_indices=torch.tensor(host_pages[:n_pages], dtype=torch.int32),

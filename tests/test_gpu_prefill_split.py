@@ -70,10 +70,12 @@ def test_scale_sign(gpu_device, scale):
     _check(out, want.float().cpu().numpy(), torch.bfloat16)
 
 
-def test_run_on_another_stream_follows_the_plan(gpu_device):
-    """The plan's upload is asynchronous: a run on a stream of its own, right
-    after plan_prefill and behind pending work on the planning stream, reads
-    the plan's tables, and a later plan's upload does not disturb it."""
+@pytest.mark.parametrize("wait", [True, False])
+def test_run_on_another_stream_follows_the_plan(gpu_device, wait):
+    """A run on a stream of its own, right after the plan and behind pending
+    work on the planning stream, reads the plan's tables, and a later plan's
+    upload does not disturb it: where the plan waits for its upload
+    (plan_prefill) and where it does not (the decoder's prefill)."""
     cases = [_case([77], [9077], 8, 2, 128, 16, torch.bfloat16, gpu_device, seed=s) for s in (1, 2)]
     want = []
     for c in cases:
@@ -84,9 +86,32 @@ def test_run_on_another_stream_follows_the_plan(gpu_device):
     big = torch.randn((4096, 4096), device=gpu_device)
     for c in cases:
         big = (big @ big).clamp_(-1, 1)  # the planning stream is busy when the upload is enqueued
-        be.plan_prefill(qo_indptr=c["qo_indptr"], paged_kv_indptr=c["indptr"], paged_kv_indices=c["indices"],
-                        paged_kv_last_page_len=c["last"])
+        be._plan_prefill(c["qo_indptr"], c["indptr"], c["indices"], c["last"], wait=wait)
         with torch.cuda.stream(side):
             got.append(be.run_prefill(c["q"], c["cache"]))
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_capture_right_after_the_plan(gpu_device):
+    """plan_prefill has uploaded its tables when it returns: a capture begun
+    without a synchronization, and replayed on a stream that waits for nothing,
+    reads them."""
+    case = _case([77], [9077], 8, 2, 128, 16, torch.bfloat16, gpu_device, seed=1)
+    want = _backend(case, 8, 2, 128, 16, gpu_device).run_prefill(case["q"], case["cache"])
+    be = _backend(case, 8, 2, 128, 16, gpu_device)
+    big, side, graph = torch.randn((4096, 4096), device=gpu_device), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    big = (big @ big).clamp_(-1, 1)  # the planning stream is busy when the upload is enqueued
+    be.plan_prefill(qo_indptr=case["qo_indptr"], paged_kv_indptr=case["indptr"], paged_kv_indices=case["indices"],
+                    paged_kv_last_page_len=case["last"])
+    assert be._prefill_plan["ready"] is None
+    with torch.cuda.stream(side):
+        graph.capture_begin()
+        got = be.run_prefill(case["q"], case["cache"])
+        graph.capture_end()
+        for _ in range(3):
+            got.zero_()
+            graph.replay()
+            side.synchronize()
+            assert torch.equal(got, want)
