@@ -737,6 +737,19 @@ extern "C" int pl_weight_unshuffle(const void* shuffled, size_t shuffled_bytes, 
   return ok();
 }
 
+int pl::wgemm::linear_rows16(const void* x, int64_t ldx, int tokens, int K, const void* W, int N, const void* bias,
+                             void* out, int64_t ldo, int dtype, hipStream_t s) {
+  const dim3 grid((N + 15) / 16, (tokens + 15) / 16);
+  if (dtype == PL_DTYPE_BF16)
+    hipLaunchKernelGGL((shuffled_gemm_kernel<bf16_t, false>), grid, dim3(kThreads), 0, s, (const bf16_t*)x, ldx,
+                       tokens, K, (const bf16_t*)W, N, (const bf16_t*)bias, (bf16_t*)out, ldo, nullptr, 0, 0);
+  else
+    hipLaunchKernelGGL((shuffled_gemm_kernel<f16_t, false>), grid, dim3(kThreads), 0, s, (const f16_t*)x, ldx, tokens,
+                       K, (const f16_t*)W, N, (const f16_t*)bias, (f16_t*)out, ldo, nullptr, 0, 0);
+  PL_LAUNCH_CHECK("shuffled_gemm_kernel");
+  return PL_OK;
+}
+
 extern "C" int pl_linear_shuffled(const void* x, int64_t ldx, int num_tokens, int in_features, const void* shuffled,
                                   int out_features, const void* bias, void* out, int64_t ldo, int dtype,
                                   void* stream) {
@@ -751,24 +764,15 @@ extern "C" int pl_linear_shuffled(const void* x, int64_t ldx, int num_tokens, in
   if (ldo < out_features) return fail(PL_ERR_INVALID, "ldo < out_features");
   if (dtype != PL_DTYPE_BF16 && dtype != PL_DTYPE_F16)
     return fail(PL_ERR_UNSUPPORTED, "pl_linear_shuffled dtype must be F16 or BF16 (got %d)", dtype);
-  // past one 16-token tile this kernel would stream W once per tile
-  if (num_tokens > 16 && wgemm::wide_supports(ldx)) {
-    const int st = wgemm::wide_linear(x, ldx, num_tokens, in_features, shuffled, out_features, bias, out, ldo, nullptr,
-                                      0, dtype, (hipStream_t)stream);
-    return st ? st : ok();
-  }
-  const dim3 grid((out_features + 15) / 16, (num_tokens + 15) / 16);
-  hipStream_t s = (hipStream_t)stream;
-  if (dtype == PL_DTYPE_BF16)
-    hipLaunchKernelGGL((shuffled_gemm_kernel<bf16_t, false>), grid, dim3(kThreads), 0, s, (const bf16_t*)x, ldx,
-                       num_tokens, in_features, (const bf16_t*)shuffled, out_features, (const bf16_t*)bias,
-                       (bf16_t*)out, ldo, nullptr, 0, 0);
-  else
-    hipLaunchKernelGGL((shuffled_gemm_kernel<f16_t, false>), grid, dim3(kThreads), 0, s, (const f16_t*)x, ldx,
-                       num_tokens, in_features, (const f16_t*)shuffled, out_features, (const f16_t*)bias,
-                       (f16_t*)out, ldo, nullptr, 0, 0);
-  PL_LAUNCH_CHECK("shuffled_gemm_kernel");
-  return ok();
+  // past one 16-token tile linear_rows16 streams W once per tile
+  int st = wgemm::kTakeRows16;
+  if (num_tokens > 16 && wgemm::wide_supports(ldx))
+    st = wgemm::wide_linear(x, ldx, num_tokens, in_features, shuffled, out_features, bias, out, ldo, nullptr, 0, dtype,
+                            (hipStream_t)stream);
+  if (st == wgemm::kTakeRows16)
+    st = wgemm::linear_rows16(x, ldx, num_tokens, in_features, shuffled, out_features, bias, out, ldo, dtype,
+                              (hipStream_t)stream);
+  return st ? st : ok();
 }
 
 extern "C" int pl_linear_shuffled_split(const void* x, int64_t ldx, int num_tokens, int in_features,

@@ -38,9 +38,15 @@ __host__ __device__ inline int split_begin(int steps, int splits, int s) {
 bool wide_supports(int64_t ldx);
 
 // out = x . W^T (+ bias); arguments checked by the caller.  ws (nullable)
-// holds a K split's planes where one pays.
+// holds a K split's planes where one pays.  kTakeRows16, and nothing done,
+// where linear_rows16 is the faster one (up to 64 tokens).
+constexpr int kTakeRows16 = -1;
 int wide_linear(const void* x, int64_t ldx, int tokens, int K, const void* W, int N, const void* bias, void* out,
                 int64_t ldo, void* ws, size_t ws_bytes, int dtype, hipStream_t s);
+
+// The decode GEMM on 16-token tiles (skinny_gemm.hip), each of which streams W.
+int linear_rows16(const void* x, int64_t ldx, int tokens, int K, const void* W, int N, const void* bias, void* out,
+                  int64_t ldo, int dtype, hipStream_t s);
 
 }  // namespace wgemm
 }  // namespace pl

@@ -427,6 +427,58 @@ static Choice choose(int tokens, int N, int K, bool allow_split) {
   return best;
 }
 
+// linear_rows16's time back to back in a graph, fitted (sd 9 %) to 864 products
+// of 33 .. 64 tokens, 1000 .. 8192 outputs, K = 1024 .. 12288: a workgroup's own
+// chain, or the rounds of 256 workgroups, of which a further token tile costs
+// less where it runs on the XCD that holds the same columns' weights
+// (consecutive workgroups go round the eight XCDs).
+static double rows16_us(int tokens, int N, int K) {
+  const int nb = (N + 15) / 16, mt = (tokens + 15) / 16;
+  const double more = mt - 1.5 + (tokens - 16 * (mt - 1)) / 32.0;  // token tiles past the first, the last by its fill
+  return 2.0 + K * 1e-3 * std::max(1.05, 0.32 + 1.95 * nb * (1 + (nb % 8 ? 0.8 : 0.55) * more) / 256);
+}
+
+// Up to 64 tokens the 16-token kernel is still the faster one for few columns:
+// its workgroups are 16 columns x 16 tokens, so all of them run at once where
+// these kernels leave CUs idle.
+struct Route {
+  bool rows16;
+  Choice c;  // tile kernel (K % 64 == 0, more than kStripMaxTokens)
+};
+static Route route(int tokens, int N, int K, bool allow_split) {
+  const int nb = (N + 15) / 16, mt = (tokens + 15) / 16;
+  if (tokens <= 16) return {true, {}};
+  // Against the strip kernel of two token tiles per workgroup, wherever the
+  // 16-token kernel is one round: 32 tokens x 1000 x 8192 12.7 us against 17.9,
+  // 1902 x 4096 8.0 against 10.2; 2854 x 4096 (358 workgroups) 13.0 against
+  // 10.3; a second tile of one token costs it a whole one (17 x 1902 x 12288
+  // 19.5 against 18.6).
+  if (tokens <= kStripMaxTokens) return {tokens >= 18 && nb * mt <= kCUs, {}};
+  // Against the strip kernel of four: one round, or two where the token tiles
+  // share the weights in an L2 (rows16_us).  64 x 1000 x 4704 10.0 us against
+  // 14.7, 2048 x 4704 10.7 against 14.6; 1902 x 4704 (476) 17.0 against 14.8.
+  if (K % 64) return {tokens <= PL_LINEAR_MAX_TOKENS && nb * mt <= (nb % 8 ? 1 : 2) * kCUs, {}};
+  Choice c = choose(tokens, N, K, allow_split);
+  if (tokens > PL_LINEAR_MAX_TOKENS) return {false, c};
+  // Against the tile kernel, by their estimates back to back (choose's are of
+  // calls alone) and by what a call takes the host, 9 us, 9.5 with a query for
+  // the workspace and 13.7 with the allocation and a split's second launch:
+  // 37 x 1902 x 2112 7.5 us against 8.6, enqueued alone 8.7 against 13.9; 37 x
+  // 1902 x 6144 17.0 against 10.2.  A split that the host would bound gives way
+  // to an unsplit call.
+  auto cost = [](double us, double host) { return std::max(us, host) + 0.01 * us; };
+  const double rows16 = cost(rows16_us(tokens, N, K), 9.0);
+  if (c.splits == 1) return {rows16 <= cost(1.46 + 0.51 * (c.us - 4), 9.5), c};
+  const double split = 0.73 + 0.82 * (c.us - 4);
+  if (rows16 <= cost(split, 13.7)) return {true, c};
+  if (split < 13.7) {
+    const Choice one = choose(tokens, N, K, false);
+    const double us = 1.46 + 0.51 * (one.us - 4);
+    if (us < 13.0 && cost(us, 9.5) <= cost(split, 13.7)) c = one;
+  }
+  return {c.splits == 1 && rows16 <= cost(1.46 + 0.51 * (c.us - 4), 9.5), c};
+}
+
 static int64_t split_ld(int N) { return (int64_t)(N + 15) / 16 * 16; }
 
 template <typename T, int I>
@@ -444,6 +496,11 @@ template <typename T>
 static int wide(const void* x, int64_t ldx, int tokens, int K, const void* W, int N, const void* bias, void* out,
                 int64_t ldo, void* ws, size_t ws_bytes, hipStream_t s) {
   const bool vec = ldo % 4 == 0 && (uintptr_t)out % 8 == 0;
+  Route r = route(tokens, N, K, true);
+  const int64_t ldp = split_ld(N);
+  if (!r.rows16 && r.c.splits > 1 && (ws == nullptr || ws_bytes < (size_t)r.c.splits * tokens * ldp * sizeof(float)))
+    r = route(tokens, N, K, false);
+  if (r.rows16) return kTakeRows16;
   if (tokens <= kStripMaxTokens || K % 64) {
     StripArgs g{x, W, bias, out, ldx, ldo, tokens, K, N, 0};
     const bool narrow = N < 32 * 128;
@@ -464,10 +521,7 @@ static int wide(const void* x, int64_t ldx, int tokens, int K, const void* W, in
     PL_LAUNCH_CHECK("strip_gemm_kernel");
     return PL_OK;
   }
-  Choice c = choose(tokens, N, K, true);
-  const int64_t ldp = split_ld(N);
-  if (c.splits > 1 && (ws == nullptr || ws_bytes < (size_t)c.splits * tokens * ldp * sizeof(float)))
-    c = choose(tokens, N, K, false);
+  const Choice& c = r.c;
   const TileShape& sh = kShapes[c.shape];
   TileArgs g{};
   g.x = x;
@@ -512,14 +566,16 @@ using namespace pl::wgemm;
 
 extern "C" size_t pl_linear_shuffled_wide_workspace_size(int num_tokens, int in_features, int out_features) {
   if (num_tokens <= kStripMaxTokens || in_features <= 0 || in_features % 64 || out_features <= 0) return 0;
-  const Choice c = choose(num_tokens, out_features, in_features, true);
-  return c.splits > 1 ? (size_t)c.splits * num_tokens * split_ld(out_features) * sizeof(float) : 0;
+  const Route r = route(num_tokens, out_features, in_features, true);
+  const Choice& c = r.c;
+  return !r.rows16 && c.splits > 1 ? (size_t)c.splits * num_tokens * split_ld(out_features) * sizeof(float) : 0;
 }
 
 extern "C" int pl_linear_shuffled_wide_splits(int num_tokens, int in_features, int out_features,
                                               int32_t* step_begin_h) {
   if (num_tokens <= kStripMaxTokens || in_features <= 0 || in_features % 64 || out_features <= 0) return 1;
-  const int splits = choose(num_tokens, out_features, in_features, true).splits;
+  const Route r = route(num_tokens, out_features, in_features, true);
+  const int splits = r.rows16 ? 1 : r.c.splits;
   for (int s = 0; s <= splits && step_begin_h != nullptr; ++s)
     step_begin_h[s] = split_begin(in_features / 64, splits, s);
   return splits;
@@ -539,15 +595,13 @@ extern "C" int pl_linear_shuffled_wide(const void* x, int64_t ldx, int num_token
   if ((uintptr_t)workspace % 16) return fail(PL_ERR_INVALID, "workspace must be 16-byte aligned");
   if (dtype != PL_DTYPE_BF16 && dtype != PL_DTYPE_F16)
     return fail(PL_ERR_UNSUPPORTED, "pl_linear_shuffled_wide dtype must be F16 or BF16 (got %d)", dtype);
-  if (!wide_supports(ldx)) {  // rows too far apart for these kernels' offsets: 64 of them at a time
-    for (int t = 0; t < num_tokens; t += PL_LINEAR_MAX_TOKENS)
-      if (const int st = pl_linear_shuffled((const char*)x + (int64_t)t * ldx * 2, ldx,
-                                            std::min(num_tokens - t, PL_LINEAR_MAX_TOKENS), in_features, shuffled,
-                                            out_features, bias, (char*)out + (int64_t)t * ldo * 2, ldo, dtype, stream))
-        return st;
-    return ok();
-  }
-  const int st = wide_linear(x, ldx, num_tokens, in_features, shuffled, out_features, bias, out, ldo, workspace,
-                             workspace_bytes, dtype, (hipStream_t)stream);
+  // (rows too far apart for these kernels' offsets: the 16-token kernel)
+  int st = kTakeRows16;
+  if (wide_supports(ldx))
+    st = wide_linear(x, ldx, num_tokens, in_features, shuffled, out_features, bias, out, ldo, workspace,
+                     workspace_bytes, dtype, (hipStream_t)stream);
+  if (st == kTakeRows16)
+    st = linear_rows16(x, ldx, num_tokens, in_features, shuffled, out_features, bias, out, ldo, dtype,
+                       (hipStream_t)stream);
   return st ? st : ok();
 }

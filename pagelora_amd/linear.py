@@ -9,6 +9,7 @@ replaces the base ``F.linear`` of the reference's projections
 
 from __future__ import annotations
 
+import functools
 import ctypes
 
 import torch
@@ -92,12 +93,33 @@ class ShuffledWeight:
                    "pl_weight_shuffle")
 
 
+@functools.lru_cache(maxsize=1024)
+def _wide_workspace(tokens: int, in_features: int, out_features: int) -> int:
+    """Bytes of workspace of a product of these sizes (0: none)."""
+    return _lib.load().pl_linear_shuffled_wide_workspace_size(tokens, in_features, out_features)
+
+
 def linear_shuffled(x: torch.Tensor, weight: ShuffledWeight, bias: torch.Tensor | None = None,
                     out: torch.Tensor | None = None) -> torch.Tensor:
     """``x . W^T (+ bias)`` for up to 64 tokens from a :class:`ShuffledWeight`."""
-    if x.dim() == 2 and x.shape[0] > _lib.PL_LINEAR_MAX_TOKENS:
+    if x.dim() != 2 or x.stride(1) != 1 or x.shape[1] != weight.in_features or x.dtype != weight.dtype:
+        raise ValueError(f"x must be [T, {weight.in_features}] of {weight.dtype} with unit column stride")
+    T, K, N = x.shape[0], weight.in_features, weight.out_features
+    if T > _lib.PL_LINEAR_MAX_TOKENS:
         raise ValueError(f"linear_shuffled takes at most {_lib.PL_LINEAR_MAX_TOKENS} tokens")
-    return linear_shuffled_wide(x, weight, bias, out)
+    if T > 32 and _wide_workspace(T, K, N):  # (no call of up to 32 tokens splits K)
+        return linear_shuffled_wide(x, weight, bias, out)
+    out = torch.empty((T, N), dtype=x.dtype, device=x.device) if out is None else out
+    if out.shape != (T, N) or out.stride(1) != 1 or out.dtype != x.dtype:
+        raise ValueError("out must be [T, out] with unit column stride")
+    if bias is not None and (bias.numel() != N or bias.dtype != x.dtype):
+        raise ValueError("bias must be [out] of x's dtype")
+    lib = _lib.load()
+    _lib.check(lib.pl_linear_shuffled(x.data_ptr(), x.stride(0), T, K, weight.data.data_ptr(), N,
+                                      bias.data_ptr() if bias is not None else None, out.data_ptr(), out.stride(0),
+                                      _lib.dtype_code(x.dtype), _lib.stream_handle(x.device)),
+               "pl_linear_shuffled")
+    return out
 
 
 def linear_shuffled_wide(x: torch.Tensor, weight: ShuffledWeight, bias: torch.Tensor | None = None,
@@ -111,17 +133,12 @@ def linear_shuffled_wide(x: torch.Tensor, weight: ShuffledWeight, bias: torch.Te
         raise ValueError("out must be [T, out] with unit column stride")
     if bias is not None and (bias.numel() != N or bias.dtype != x.dtype):
         raise ValueError("bias must be [out] of x's dtype")
-    lib = _lib.load()
-    bias_ptr = bias.data_ptr() if bias is not None else None
-    if T <= 16:
-        _lib.check(lib.pl_linear_shuffled(x.data_ptr(), x.stride(0), T, K, weight.data.data_ptr(), N, bias_ptr,
-                                          out.data_ptr(), out.stride(0), _lib.dtype_code(x.dtype),
-                                          _lib.stream_handle(x.device)), "pl_linear_shuffled")
-        return out
-    nbytes = lib.pl_linear_shuffled_wide_workspace_size(T, K, N)
+    nbytes = _wide_workspace(T, K, N)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
-    _lib.check(lib.pl_linear_shuffled_wide(x.data_ptr(), x.stride(0), T, K, weight.data.data_ptr(), N, bias_ptr,
-                                           out.data_ptr(), out.stride(0), ws.data_ptr() if nbytes else None, nbytes,
+    lib = _lib.load()
+    _lib.check(lib.pl_linear_shuffled_wide(x.data_ptr(), x.stride(0), T, K, weight.data.data_ptr(), N,
+                                           bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                                           out.stride(0), ws.data_ptr() if nbytes else None, nbytes,
                                            _lib.dtype_code(x.dtype), _lib.stream_handle(x.device)),
                "pl_linear_shuffled_wide")
     return out

@@ -44,13 +44,22 @@ def test_linear_wide_vs_oracle(gpu_device, dtype, tokens, n, k):
     assert (err <= 2e-3 + REL[dtype] * np.abs(want)).all(), f"max err {err.max():.3e}"
 
 
-# K steps that their splits do not divide evenly (33, 42, 65 by 8, 19 by 4, 33 by 2)
+# K steps that their splits do not divide evenly (33, 42, 65 by 8, 55 and 27 by 4, 69 by 2)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("tokens,n,k,splits", [(48, 1000, 2112, 8), (64, 4096, 2688, 8), (65, 1000, 4160, 8),
-                                               (49, 37, 1216, 4), (40, 8208, 2112, 2)])
+@pytest.mark.parametrize("tokens,n,k,splits", [(65, 1000, 2112, 8), (65, 1000, 2688, 8), (65, 1000, 4160, 8),
+                                               (33, 4112, 3520, 4), (77, 4096, 1728, 4), (77, 8208, 4416, 2)])
 def test_uneven_splits(gpu_device, dtype, tokens, n, k, splits):
     assert _lib.load().pl_linear_shuffled_wide_splits(tokens, k, n, None) == splits
     test_linear_wide_vs_oracle(gpu_device, dtype, tokens, n, k)
+
+
+# Up to 64 tokens, either side of where the 16-token kernel takes over: one
+# round of workgroups, two that share weights, an unsplit product of few steps
+@pytest.mark.parametrize("tokens,n,k", [(18, 2048, 160), (18, 2064, 160), (32, 2040, 4704), (33, 1360, 96),
+                                        (33, 1376, 96), (64, 2048, 352), (64, 2064, 352), (64, 1000, 1024),
+                                        (40, 8192, 1280), (33, 4096, 1600), (56, 2300, 3072)])
+def test_few_columns(gpu_device, tokens, n, k):
+    test_linear_wide_vs_oracle(gpu_device, torch.bfloat16, tokens, n, k)
 
 
 def test_strided_x_without_workspace(gpu_device):
