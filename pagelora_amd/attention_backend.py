@@ -638,7 +638,8 @@ class PagedDecodeAttention:
             "causal": bool(causal),
             "max_page": max_page,
             "tables": (*tables_d, items_d),
-            "stream": stream,
+            "table_ptrs": [t.data_ptr() for t in (*tables_d, items_d)],
+            "stream": stream.cuda_stream,
             # of an upload not waited for: a run on another stream waits for it
             "ready": None if wait else ready,
             "q_data_type": q_data_type,
@@ -686,12 +687,12 @@ class PagedDecodeAttention:
             raise ValueError(f"q dtype {q.dtype} != KV cache dtype {k.dtype}")
         if plan["max_page"] >= num_pages:
             raise ValueError(f"page id {plan['max_page']} is outside the {num_pages}-page KV pool")
-        qo_d, kv_d, ind_d, last_d, items_d = plan["tables"]
-        stream = torch.cuda.current_stream(q.device)
+        stream = _lib.stream_handle(q.device)
         if stream != plan["stream"] and not torch.cuda.is_current_stream_capturing():
+            here = torch.cuda.current_stream(q.device)
             if plan["ready"] is not None:
-                stream.wait_event(plan["ready"])
-            qo_d.record_stream(stream)  # one allocation holds every table
+                here.wait_event(plan["ready"])
+            plan["tables"][0].record_stream(here)  # one allocation holds every table
         if plan["split"]:
             # per call, from torch's allocator: calls on other streams share nothing
             nbytes = plan["workspace_bytes"]
@@ -700,12 +701,11 @@ class PagedDecodeAttention:
                 q.data_ptr(), q.stride(0), q.stride(1),
                 k.data_ptr(), v.data_ptr(), page_stride, token_stride, head_stride,
                 num_pages,
-                qo_d.data_ptr(), kv_d.data_ptr(), ind_d.data_ptr(), last_d.data_ptr(),
-                items_d.data_ptr(), plan["num_items"], plan["num_merges"],
+                *plan["table_ptrs"], plan["num_items"], plan["num_merges"],
                 out.data_ptr(), out.stride(0), out.stride(1),
                 plan["batch"], self.num_qo_heads, self.num_kv_heads, self.page_size,
                 int(plan["causal"]), self.sm_scale, ws.data_ptr() if nbytes else None, nbytes, nbytes,
-                _lib.dtype_code(q.dtype), _lib.stream_handle(q.device),
+                _lib.dtype_code(q.dtype), stream,
             )
             _lib.check(status, "pl_prefill_split_run")
             return out
@@ -713,12 +713,11 @@ class PagedDecodeAttention:
             q.data_ptr(), q.stride(0), q.stride(1),
             k.data_ptr(), v.data_ptr(), page_stride, token_stride, head_stride,
             num_pages,
-            qo_d.data_ptr(), kv_d.data_ptr(), ind_d.data_ptr(), last_d.data_ptr(),
-            items_d.data_ptr(), plan["num_items"],
+            *plan["table_ptrs"], plan["num_items"],
             out.data_ptr(), out.stride(0), out.stride(1),
             plan["batch"], self.num_qo_heads, self.num_kv_heads, self.head_dim, self.page_size,
             int(plan["causal"]), self.sm_scale, _lib.dtype_code(q.dtype),
-            _lib.stream_handle(q.device),
+            stream,
         )
         _lib.check(status, "pl_prefill_run")
         return out
