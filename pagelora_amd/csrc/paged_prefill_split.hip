@@ -525,12 +525,17 @@ extern "C" int pl_prefill_split_plan(const int32_t* qo_indptr_h, const int32_t* 
     }
   }
   if (list.size() > (size_t)INT32_MAX / 64) return fail(PL_ERR_INVALID, "too many prefill work items");
-  // A part's length: an even share of the work per slot, if the longest row
-  // item is more than twice that (2119 tokens MHA, 1.7 times: 56.5 us whole,
-  // 68 cut; 77 behind 32000, 21 times: 77 us in 504 parts, 114 in 252, 87 in
-  // 1000).
+  // A part's length: an even share of the work per slot.  Ranges are cut where
+  // the longest row item is more than twice that, and by four tiles more, which
+  // the partial results and the merge cost: 2119 tokens MHA (34 tiles, share
+  // 20) 56.5 us whole, 68 cut; 3 x 300 behind 300 GQA 4 (10, 4) 23.2 whole, 42.6
+  // cut; 3 x 300 behind 1500 (29, 13) 51.3 whole, 71.0 cut; 500 behind 800 (21,
+  // 5) 39.5 whole, 33.6 cut; 77 behind 32000 (501, 16) 700 whole, 77 cut.  Over
+  // 624 calls of 1 to 3 requests of 2 to 2200 tokens behind 0 to 30000 the
+  // choice is 5 % from the better of the two in the mean, without the four
+  // tiles 6.3 %, with eight 6.9.
   const int64_t share = std::max<int64_t>(kMinTiles, (work * num_kv_heads + kSlots - 1) / kSlots);
-  const int64_t chunk = longest > 2 * share ? share : INT32_MAX;
+  const int64_t chunk = longest > 2 * share + 4 ? share : INT32_MAX;
   std::vector<Item> items, merges;
   int slots = 0;
   for (const Rows& e : list) {
