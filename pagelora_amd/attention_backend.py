@@ -104,6 +104,27 @@ def _upload_int32(host: "Sequence[torch.Tensor]", device: torch.device) -> list[
     return [buf[at:at + t.numel()] for t, at in zip(host, starts)]
 
 
+def _prefill_rows64(qo_lens: list[int], kv_lens: list[int], num_qo_heads: int, num_kv_heads: int) -> bool:
+    """Whether the 64-row prefill kernel is the faster one at head_dim 128:
+    short sequences, whose few tiles the split kernel's longer fill outlasts,
+    while its 128-row items leave CUs idle, or where they are padding to a
+    sixth and more.  us, 64-row kernel against split kernel, in a graph: 27
+    tokens (7 heads per kv head) 5.5, 8.1; 16 x 64 tokens of the same 8, 9.5;
+    128 x 17 tokens MHA 29, 48; 128 x 300 tokens MHA 370, 462.  Past the bounds:
+    4 x 256 tokens GQA 4 18, 15.5; 4 x 300 tokens MHA 23, 17.6; 300 behind 200
+    MHA 21, 19.4."""
+    g = num_qo_heads // num_kv_heads
+    tiles = -(-max(kv_lens, default=0) // 64)
+    if tiles > 5:
+        return False
+    items64 = sum(-(-n * g // 64) for n in qo_lens)
+    items128 = sum(-(-n * g // 128) for n in qo_lens)
+    groups = items64 * num_kv_heads
+    if tiles <= 4 and groups <= (512 if tiles <= 2 else 256):
+        return True
+    return items128 * 2 >= 1.2 * items64 and (tiles <= 2 or groups >= 5120)
+
+
 def _cache_geometry(cache, num_kv_heads: int, head_dim: int, page_size: int):
     """(k_tensor, v_tensor_or_ptr_source, page_stride, token_stride, head_stride, num_pages)."""
 
@@ -606,8 +627,14 @@ class PagedDecodeAttention:
         args = (qo_h.data_ptr(), kv_h.data_ptr(), last_h.data_ptr(), batch, self.num_qo_heads, self.num_kv_heads,
                 self.page_size, int(bool(causal)))
         # the split-range kernel is built for head_dim 128 and loads four
-        # tokens of a page at a time; the 64-row kernel takes the rest
+        # tokens of a page at a time; the 64-row kernel takes the rest, and the
+        # calls that it is faster at
         split = self.head_dim == 128 and self.page_size % 4 == 0
+        if split:
+            qo, kv = qo_h.tolist(), kv_h.tolist()
+            kv_lens = [(b - a - 1) * self.page_size + n for a, b, n in zip(kv, kv[1:], last_h.tolist()) if b > a]
+            split = not _prefill_rows64([b - a for a, b in zip(qo, qo[1:])], kv_lens, self.num_qo_heads,
+                                        self.num_kv_heads)
         if split:
             counts = (ctypes.byref(n), ctypes.byref(merges), ctypes.byref(ws_bytes))
             _lib.check(self._lib.pl_prefill_split_plan(*args, None, 0, *counts), "pl_prefill_split_plan")

@@ -46,11 +46,30 @@ def test_long_range_is_cut_and_equals_whole(gpu_device):
     _check(out, _oracle(case), torch.float16)
 
 
+# either side of where the 64-row kernel takes short sequences
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,qo_lens,kv_lens,split", [
+    ((4, 1), [1], [1], False), ((7, 1), [64, 17], [256, 17], False), ((7, 1), [64, 17], [257, 17], True),
+    ((8, 8), [128] * 16, [128] * 16, False),   # 256 workgroups
+    ((8, 8), [128] * 17, [129] * 17, True),    # 272 of three tiles
+    ((32, 32), [17] * 20, [17] * 20, False),   # 640, half of the 128-row items padding
+    ((32, 32), [128] * 9, [128] * 9, True),
+])
+def test_short_sequences(gpu_device, dtype, heads, qo_lens, kv_lens, split):
+    case = _case(qo_lens, kv_lens, *heads, 128, 16, dtype, gpu_device, seed=len(qo_lens))
+    be = _backend(case, *heads, 128, 16, gpu_device)
+    assert be._prefill_plan["split"] == split
+    out = be.run_prefill(case["q"], case["cache"])
+    torch.cuda.synchronize()
+    _check(out, _oracle(case), dtype)
+
+
 @pytest.mark.parametrize("scale", [-0.05, 0.0])
 def test_scale_sign(gpu_device, scale):
     """A negative or zero softmax scale: the same as the 64-row kernel on pages of 2 tokens."""
-    case = _case([50], [200], 4, 2, 128, 16, torch.bfloat16, gpu_device, seed=2)
+    case = _case([50, 3], [200, 400], 4, 2, 128, 16, torch.bfloat16, gpu_device, seed=2)
     be = _backend(case, 4, 2, 128, 16, gpu_device)
+    assert be._prefill_plan["split"]
     be.sm_scale = scale
     out = be.run_prefill(case["q"], case["cache"])
     pages = case["indices"].long()
@@ -61,8 +80,10 @@ def test_scale_sign(gpu_device, scale):
     ref = PagedDecodeAttention(device=gpu_device, workspace_mb=8, num_qo_heads=4, num_kv_heads=2, head_dim=128,
                                page_size=2)
     i32 = lambda x: torch.tensor(x, dtype=torch.int32)  # noqa: E731
-    ref.plan_prefill(qo_indptr=i32([0, 50]), paged_kv_indptr=i32([0, 100]),
-                     paged_kv_indices=torch.arange(100, dtype=torch.int32), paged_kv_last_page_len=i32([2]))
+    # 200 tokens are 13 pages of 16, the last of 8; 400 are 25 whole ones
+    order = torch.cat([torch.arange(100), torch.arange(104, 304)]).to(torch.int32)
+    ref.plan_prefill(qo_indptr=i32([0, 50, 53]), paged_kv_indptr=i32([0, 100, 300]), paged_kv_indices=order,
+                     paged_kv_last_page_len=i32([2, 2]))
     assert not ref._prefill_plan["split"]
     ref.sm_scale = scale
     want = ref.run_prefill(case["q"], small.to(gpu_device))
