@@ -259,6 +259,7 @@ __device__ __forceinline__ void load8_planes(const SplitIn& sp, int64_t t, int c
 constexpr int kRowNormMaxHidden = 8192;
 constexpr int kNormRows = 2;       // rows per workgroup of add_rmsnorm_rows_kernel
 constexpr int kNormRowsMin = 320;  // from these rows on
+constexpr int kNormRowsMinB = 8192;  // ... and hidden x rank
 
 // YS: the module's y comes from ys.splits fp32 side planes (the LoRA A rows
 // of pl_linear_shuffled_side, column y_offset + a*R of each plane): thread
@@ -384,6 +385,8 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_row_kernel(
 // 16) out of the L2 for every row, which bounds it past a few hundred rows:
 // 384 rows 6.1 -> 5.3 us, 1024 10.7 -> 9.1, 2112 21.0 -> 16.4; 256 rows 4.7
 // against 5.0.  Four rows leave too few workgroups (384 rows 7.1, 2112 16.6).
+// A B of few columns is cheap to read again: rank 8, 512 rows x 256 3.68 us
+// against 3.72, x 64 3.5, 3.7, x 1024 4.6, 4.3.
 template <typename T, int R, int N>
 __global__ __launch_bounds__(512) void add_rmsnorm_rows_kernel(
     T* __restrict__ r, int64_t ldr, const T* __restrict__ x, int64_t ldx, const T* __restrict__ w,
@@ -881,7 +884,7 @@ static int launch_norm(bool add, int rank, void* r, int64_t ldr, const void* x, 
   if constexpr (sizeof(T) == 2) {
     // decode-sized rows: the single-chunk kernel (two memory round trips)
     if (add && xs.splits == 0 && (rank == 8 || rank == 16) && lu.adapter >= 0 && rows >= kNormRowsMin &&
-        hidden <= 4096) {
+        hidden <= 4096 && hidden * rank >= kNormRowsMinB) {
       const int threads = (hidden / 8 + kWave - 1) / kWave * kWave;
       auto go = [&](auto rk) {
         constexpr int R = decltype(rk)::value;
@@ -1073,7 +1076,7 @@ static int silu_common(const void* gate_up, int64_t ldg, void* out, int64_t ldo,
     rank = lg.rank;
   }
   hipStream_t s = (hipStream_t)stream;
-  if (rank > 0 && dtype != PL_DTYPE_F32 && prompt::takes(rows, lg) && rows <= 32 * 65535) {
+  if (rank > 0 && dtype != PL_DTYPE_F32 && prompt::takes_silu(rows, inter, lg) && rows <= 32 * 65535) {
     prompt::silu_mul(gate_up, ldg, out, ldo, rows, inter, lg, lu, dtype == PL_DTYPE_BF16, s);
     PL_LAUNCH_CHECK("silu_mul_tile_kernel");
     return ok();

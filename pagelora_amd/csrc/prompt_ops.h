@@ -7,15 +7,22 @@
 namespace pl {
 namespace prompt {
 
-// From these rows on the tokens share their adapter's B rows through MFMA
-// tiles; fewer take the row kernels, which read B once per token.
-// SiLU*up x 12288, row kernel -> tiles: 24 rows 5.8 -> 5.5 us, 64 8.6 -> 5.6,
-// 256 26.5 -> 8.7, 2112 264 -> 40.
-constexpr int kMinRows = 24;
-// q/k norm + RoPE + append, 48 heads: 2112 rows 45 -> 21 us, 512 rows 16.8 ->
-// 13.9, but a tile's chain of three heads costs 11 us where the row kernel
-// takes 5.5 (77 rows).
+// Where the tokens share their adapter's B rows through MFMA tiles; elsewhere
+// the row kernels, which read B once per token.
+// SiLU*up: a call of the tiles takes 5.2 us at least, the row kernel 3.8 where
+// it fills no CU; the line is where its reads of B pass that.  us, row kernel
+// against tiles, rank 16 (8): 100 x 2048 5.2, 5.8 (4.3, 5.7); 24 x 11008 6.2,
+// 5.8 (4.9, 5.7); 64 x 12288 10.9, 6.1 (7.5, 6.0); 2112 x 12288 243, 37.5; many
+// rows of few columns launch many workgroups: 1000 x 64 7.2, 5.4 (6.2, 5.3).
+// Rank 32's two passes over B: 24 x 64 8.0, 5.1.
+constexpr int kMinRows = 24, kManyRows = 1000;
+constexpr int64_t kMinSiluB = 4 << 20;  // rows x columns x rank
+// q/k norm + RoPE + append: a tile's chain of three heads costs 11 us.  Rank 16
+// (8): 512 rows x 36 heads 14.3, 14.4 (14.0, 14.4); 600 x 36 16.3, 14.7 (15.5,
+// 15.0); 1000 x 6 10.1, 12.4; 2112 x 48 48.1, 23.9.  Rank 32: 1000 x 6 11.6,
+// 11.8.
 constexpr int kMinQkrRows = 512;
+constexpr int64_t kMinQkrHeads = 18000, kMinQkrHeads32 = 6000;  // rows x heads
 
 struct QkrTileArgs {
   const void *qkv, *qn, *kn;
@@ -29,9 +36,11 @@ struct QkrTileArgs {
   LoraUp m[3];
 };
 
-// Whether the tile kernels take a call's modules.
-inline bool takes(int rows, const LoraUp& m) {
-  return rows >= kMinRows && m.adapter >= 0 && (m.rank == 8 || m.rank == 16 || m.rank == 32);
+// Whether the tile kernels take a call's modules, and SiLU*up's sizes ...
+inline bool takes(const LoraUp& m) { return m.adapter >= 0 && (m.rank == 8 || m.rank == 16 || m.rank == 32); }
+inline bool takes_silu(int rows, int inter, const LoraUp& m) {
+  return takes(m) && rows >= kMinRows &&
+         (m.rank == 32 || rows >= kManyRows || (int64_t)rows * inter * m.rank >= kMinSiluB);
 }
 // ... and the q/k norm + RoPE + append's layout: head_dim 128, 16-byte chunks everywhere.
 bool takes_qkr(const QkrTileArgs& a, int head_dim);

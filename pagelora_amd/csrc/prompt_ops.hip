@@ -232,7 +232,8 @@ bool takes_qkr(const QkrTileArgs& a, int head_dim) {
   for (const void* p : ptrs)
     if ((uintptr_t)p % 16) return false;
   return head_dim == kD && a.ld % 8 == 0 && a.ps % 8 == 0 && a.ts % 8 == 0 && a.hs % 8 == 0 &&
-         a.rows >= kMinQkrRows && takes(a.rows, a.m[0]);
+         a.rows >= kMinQkrRows && takes(a.m[0]) &&
+         (int64_t)a.rows * (a.hq + 2 * a.hkv) >= (a.m[0].rank == 32 ? kMinQkrHeads32 : kMinQkrHeads);
 }
 
 void qk_norm_rope_append(const QkrTileArgs& a, bool bf16, hipStream_t s) {

@@ -32,7 +32,7 @@ def _module(gen, rows, n, width, rank, dtype, device, y, y_offset):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rank", [8, 16, 32])
-@pytest.mark.parametrize("rows", [24, 33, 101])
+@pytest.mark.parametrize("rows", [24, 33, 101, 1003])
 @pytest.mark.parametrize("inter", [8, 264, 1024])
 def test_silu_mul(gpu_device, dtype, rank, rows, inter):
     gen = torch.Generator().manual_seed(rows + inter + rank)
@@ -48,7 +48,8 @@ def test_silu_mul(gpu_device, dtype, rank, rows, inter):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rank", [8, 16, 32])
-@pytest.mark.parametrize("rows,hq,hkv,norm", [(512, 7, 1, True), (600, 32, 8, True), (527, 4, 4, False)])
+@pytest.mark.parametrize("rows,hq,hkv,norm", [(512, 7, 1, True), (600, 32, 8, True), (527, 4, 4, False),
+                                              (2001, 7, 1, True), (1503, 4, 4, False)])
 def test_qk_norm_rope_append(gpu_device, dtype, rank, rows, hq, hkv, norm):
     gen = torch.Generator().manual_seed(rows + hq + rank)
     n, D, ps = 2, 128, 16
@@ -59,13 +60,14 @@ def test_qk_norm_rope_append(gpu_device, dtype, rank, rows, hq, hkv, norm):
             for j, w in enumerate(outs_w)]
     wq, wk = ((1 + 0.1 * torch.randn(D, generator=gen)).to(dtype).to(gpu_device) if norm else None for _ in range(2))
     pos = torch.randint(0, 40000, (rows,), generator=gen)
-    slots = torch.randperm(40 * ps, generator=gen)[:rows]
+    pages = 40 if rows <= 600 else 130
+    slots = torch.randperm(pages * ps, generator=gen)[:rows]
     page, off = slots // ps, slots % ps
     page[3], off[5] = -1, ps  # outside the pool: skipped
     ids = torch.ones(rows, dtype=torch.int32, device=gpu_device)
     results = []
     for j in range(2):
-        cache = torch.zeros((40, 2, ps, hkv, D), dtype=dtype, device=gpu_device)
+        cache = torch.zeros((pages, 2, ps, hkv, D), dtype=dtype, device=gpu_device)
         q = fused_ops.qk_norm_rope_append(
             qkv[:, :width], wq, wk, pos.to(gpu_device), page.to(gpu_device), off.to(gpu_device), cache,
             num_qo_heads=hq, num_kv_heads=hkv, head_dim=D, page_size=ps, rope_theta=1e6,
@@ -79,7 +81,7 @@ def test_qk_norm_rope_append(gpu_device, dtype, rank, rows, hq, hkv, norm):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rank", [8, 16])
-@pytest.mark.parametrize("rows,hidden", [(320, 8), (321, 520), (1027, 4096), (323, 4088)])
+@pytest.mark.parametrize("rows,hidden", [(320, 8), (321, 520), (1027, 4096), (323, 4088), (321, 1032)])
 @pytest.mark.parametrize("chunk8", [False, True])
 def test_add_rmsnorm_rows(gpu_device, dtype, rank, rows, hidden, chunk8):
     """Rows sharing B in registers vs a row per workgroup."""
