@@ -1076,7 +1076,7 @@ static int silu_common(const void* gate_up, int64_t ldg, void* out, int64_t ldo,
     rank = lg.rank;
   }
   hipStream_t s = (hipStream_t)stream;
-  if (rank > 0 && dtype != PL_DTYPE_F32 && prompt::takes_silu(rows, inter, lg) && rows <= 32 * 65535) {
+  if (rank > 0 && (dtype == PL_DTYPE_BF16 || dtype == PL_DTYPE_F16) && prompt::takes_silu(rows, inter, lg) && rows <= 32 * 65535) {
     prompt::silu_mul(gate_up, ldg, out, ldo, rows, inter, lg, lu, dtype == PL_DTYPE_BF16, s);
     PL_LAUNCH_CHECK("silu_mul_tile_kernel");
     return ok();
@@ -1257,7 +1257,8 @@ static int qkr_common(const void* qkv, int64_t ld_qkv, const void* q_norm_weight
                                 v_cache, page_stride, token_stride, head_stride, num_pages, page_size, batch,
                                 num_qo_heads, num_kv_heads, inv_freq, eps,
                                 {a.lora.m[0], a.lora.m[1], a.lora.m[2]}};
-    if (xs.splits == 0 && dtype != PL_DTYPE_F32 && prompt::takes_qkr(t, head_dim) && batch <= 16 * 65535) {
+    if (xs.splits == 0 && (dtype == PL_DTYPE_BF16 || dtype == PL_DTYPE_F16) && prompt::takes_qkr(t, head_dim) &&
+        batch <= 16 * 65535) {
       prompt::qk_norm_rope_append(t, dtype == PL_DTYPE_BF16, (hipStream_t)stream);
       PL_LAUNCH_CHECK("qkr_tile_kernel");
       return ok();
