@@ -1076,7 +1076,8 @@ static int silu_common(const void* gate_up, int64_t ldg, void* out, int64_t ldo,
     rank = lg.rank;
   }
   hipStream_t s = (hipStream_t)stream;
-  if (rank > 0 && (dtype == PL_DTYPE_BF16 || dtype == PL_DTYPE_F16) && prompt::takes_silu(rows, inter, lg) && rows <= 32 * 65535) {
+  if (rank > 0 && (dtype == PL_DTYPE_BF16 || dtype == PL_DTYPE_F16) && prompt::takes_silu(rows, inter, lg) &&
+      rows <= 32 * 65535) {
     prompt::silu_mul(gate_up, ldg, out, ldo, rows, inter, lg, lu, dtype == PL_DTYPE_BF16, s);
     PL_LAUNCH_CHECK("silu_mul_tile_kernel");
     return ok();
