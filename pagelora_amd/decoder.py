@@ -211,7 +211,7 @@ class LayerWeights:
 
     def __getattr__(self, name: str):
         # w_<proj>_ext / w_<proj> of a single-copy layer: unshuffled on demand
-        # (a fresh tensor; the hot paths use the shuffled copy or row_major())
+        # (a fresh tensor; the hot paths use the shuffled copy)
         if name.startswith("w_") and self.__dict__.get("single_copy"):
             proj = name[2:-4] if name.endswith("_ext") else name[2:]
             sw = self.__dict__["shuffled"].get(proj)
@@ -527,31 +527,8 @@ def _project(x: torch.Tensor, lw: LayerWeights, name: str) -> "torch.Tensor | Sp
                 return linear_shuffled_split(x, sw, splits)
             return linear_shuffled(x, sw)
         if name in ("qkv", "o"):
-            return lora_linear(x, row_major(lw, name), None, None)
-    return F.linear(x, row_major(lw, name))
-
-
-_ROW_MAJOR_SCRATCH: dict = {}
-
-
-def row_major(lw: LayerWeights, name: str) -> torch.Tensor:
-    """The row-major [W; A] weight of projection ``name`` for a library GEMM:
-    the stored tensor, or for a single-copy layer the shuffled copy
-    unshuffled into a buffer shared by every projection of the device (stream
-    ordered: each use is enqueued after the previous one's GEMM)."""
-    if not lw.single_copy:
-        return getattr(lw, f"w_{name}_ext")
-    return unshuffled_scratch(lw.shuffled[name])
-
-
-def unshuffled_scratch(sw: ShuffledWeight) -> torch.Tensor:
-    """``sw`` unshuffled into the per-device row-major scratch buffer."""
-    key = (sw.data.device, sw.dtype)
-    need = sw.out_features * sw.in_features
-    buf = _ROW_MAJOR_SCRATCH.get(key)
-    if buf is None or buf.numel() < need:
-        buf = _ROW_MAJOR_SCRATCH[key] = torch.empty(need, dtype=sw.dtype, device=sw.data.device)
-    return sw.unshuffle(buf[:need].view(sw.out_features, sw.in_features))
+            return lora_linear(x, getattr(lw, f"w_{name}_ext"), None, None)
+    return F.linear(x, getattr(lw, f"w_{name}_ext"))
 
 
 def _cols(out, n: int):

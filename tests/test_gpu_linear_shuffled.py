@@ -195,11 +195,8 @@ def test_linear_shuffled_decoder_shapes(gpu_device, shape, tokens):
 def test_unshuffle_inverts_the_shuffle(gpu_device, shape, dtype):
     """pl_weight_unshuffle(pl_weight_shuffle(W)) == W bit for bit at the
     decoder's shapes (qkv, gate_up and down with their A rows, the lm_head)
-    and a ragged one, into a fresh tensor and into the decoder's shared
-    row-major scratch buffer (which the stage check's oracle weights and
-    prefill's library GEMMs read)."""
-    from pagelora_amd.decoder import unshuffled_scratch
-
+    and a ragged one, into a fresh tensor and into given ones (contiguous and
+    row-strided)."""
     n, k = shape
     print(f"[unshuffle] {n} x {k} {dtype}", flush=True)
     g = torch.Generator(device=gpu_device).manual_seed(n * 3 + k)
@@ -208,8 +205,9 @@ def test_unshuffle_inverts_the_shuffle(gpu_device, shape, dtype):
     fresh = sw.unshuffle()
     assert torch.equal(fresh.view(torch.int16), w.view(torch.int16))
     del fresh
-    scratch = unshuffled_scratch(sw)
-    assert torch.equal(scratch.view(torch.int16), w.view(torch.int16))
+    given = torch.zeros((n, k), dtype=dtype, device=gpu_device)
+    assert sw.unshuffle(given) is given
+    assert torch.equal(given.view(torch.int16), w.view(torch.int16))
     # a row-strided target (the unshuffle writes only the [n, k] view)
     wide = torch.full((n, k + 64), 3.0, dtype=dtype, device=gpu_device)
     sw.unshuffle(wide[:, :k])

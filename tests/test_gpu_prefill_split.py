@@ -36,14 +36,29 @@ def test_edges_vs_oracle(gpu_device, dtype, page_size, heads, qo_lens, kv_lens, 
     _check(out, _oracle(case, causal), dtype)
 
 
-def test_long_range_is_cut_and_equals_whole(gpu_device):
-    """77 queries behind 9000 tokens: parts of the kv range agree with the 64-row kernel's whole one."""
+def test_long_range_is_cut(gpu_device):
+    """77 queries behind 9000 tokens: the kv range is cut, and its parts merge to the oracle's result."""
     case = _case([77], [9077], 8, 2, 128, 16, torch.float16, gpu_device, seed=1)
     be = _backend(case, 8, 2, 128, 16, gpu_device)
     assert be._prefill_plan["num_merges"] > 0
     out = be.run_prefill(case["q"], case["cache"])
     torch.cuda.synchronize()
     _check(out, _oracle(case), torch.float16)
+
+
+# the merge takes 64 parts a pass and eight loads at a time
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,kv_len,parts", [((7, 1), 20002, 79), ((28, 4), 32002, 126), ((2, 2), 16385, 65)])
+def test_more_parts_than_a_pass(gpu_device, dtype, heads, kv_len, parts):
+    """Two queries behind a long prefix: one row item in more than 64 parts."""
+    case = _case([2], [kv_len], *heads, 128, 16, dtype, gpu_device, seed=parts)
+    be = _backend(case, *heads, 128, 16, gpu_device)
+    plan = be._prefill_plan
+    records = plan["tables"][-1].view(-1, 8).cpu()
+    assert plan["num_items"] == parts and records[plan["num_items"]:, 6].tolist() == [parts]
+    out = be.run_prefill(case["q"], case["cache"])
+    torch.cuda.synchronize()
+    _check(out, _oracle(case), dtype)
 
 
 # either side of where the 64-row kernel takes short sequences
