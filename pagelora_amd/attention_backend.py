@@ -47,9 +47,15 @@ from . import _lib
 #     (bf16, 8 kv heads: 64 x 2048 90.9 us against 92.0 at 256 items,
 #     128 x 2048 166.6 vs 170.8, 64 x 8192 325.1 vs 326.1; 192 items, an
 #     uneven count of waves per SIMD, 105.7 / 170.2 / 382.1);
-#   - other larger batches with 8 kv heads: 256 items (64 x 2048 GQA 4 on
-#     the VALU scores: 99 us against 118 us at 1,024 items; ragged
+#   - other larger batches with fewer than 16 kv heads: 256 items (64 x 2048
+#     GQA 4 on the VALU scores: 99 us against 118 us at 1,024 items; ragged
 #     64 x U[128, 8192]: 204 vs 217 us);
+#   - groups of 5 to 8 heads on the matrix wave, bf16, back to back in a graph,
+#     at 64 / 128 / 192 / 256 / 384 items: 64 x 2048 of 7 heads (4 kv) 83.3 / 50.2
+#     / 57.6 / 50.6 / 52.6 us, of 5 (8 kv) 87.8 / 92.9 / 91.4 / 91.6 / 98.1, of 8
+#     (8 kv) 89.3 / 94.0 / 93.4 / 94.6 / 104; 23 ragged rows to 4099 of 7 heads
+#     35.5 / 25.0 / 25.5 / 23.5 / 25.6, 4 x 2048 of 7 12.8 / 10.7 / 11.7 / 11.7 /
+#     11.8: the counts above are within 7 % of the best;
 #   - larger batches with >= 16 kv heads: 192 items, i.e. 6 waves per SIMD
 #     (ragged batch-64 MHA: 713.5 us against 729 us at 256 items).
 _ENV_TARGET_WAVES = os.environ.get("PAGELORA_DECODE_TARGET_WAVES")
