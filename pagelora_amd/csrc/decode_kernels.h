@@ -422,7 +422,8 @@ template <> struct ProbPlanes<f16_t> {
 // 53.7 -> 30.0 us (106 MB); 4 heads, whose P . V alone was on the VALU: 1 x
 // 2048 11.3 -> 9.75 us, 4 x 2112 15.7 -> 13.5, 1 x 32000 32.7 -> 29.2, 64 x
 // 2048 98.5 -> 96.0, the four-layer decode step 429 -> 423 (with the
-// accumulators in VGPRs; in AGPRs 0.2 to 0.7 us slower).
+// accumulators in VGPRs; in AGPRs 0.2 to 0.7 us slower).  Those are with two
+// planes of P; what the third costs stands at ProbPlanes.
 template <typename T, int D, int G>
 struct DecodeWaveMatrix {
   static_assert(D == 128 && G <= 16 && sizeof(T) == 2, "P . V on MFMA: head_dim 128, 16-bit");

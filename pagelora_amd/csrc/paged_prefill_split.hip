@@ -19,11 +19,11 @@
 // merge_kernel combines a row's parts in order.
 //
 // Bound by the matrix and vector units' shared issue: 8192 tokens of 32768
-// (GQA 4, bf16) 7885 us with 64-row items and 16 rows per wave -> 4490 us, the
-// MFMAs busy 58 % of the cycles (bf16's P is two planes, a third of them).
-// One wave's softmax beside its own neighbouring half tiles' MFMAs (software
-// pipelining) was slower (5190 us): two waves per SIMD overlap already, and
-// its registers spill.
+// (GQA 4, bf16) 7770 us with 64-row items and 16 rows per wave -> 4600 us (4410
+// a launch in a kernel trace), the MFMAs busy 58 % of the cycles (bf16's P is
+// two planes, a third of them).  One wave's softmax beside its own
+// neighbouring half tiles' MFMAs (software pipelining) was slower (5190 us):
+// two waves per SIMD overlap already, and its registers spill.
 #include <algorithm>
 #include <type_traits>
 #include <vector>
