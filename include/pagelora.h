@@ -779,9 +779,9 @@ int pl_linear_shuffled(const void* x, int64_t ldx, int num_tokens,
 size_t pl_linear_shuffled_wide_workspace_size(int num_tokens, int in_features, int out_features);
 /*
  * The K split of a call with that workspace: returns the number of splits (1:
- * unsplit).  Where in_features is a multiple of 64 and num_tokens > 32,
- * step_begin_h (nullable, room for 9) receives each split's first 64-wide
- * step of K, then the number of steps.
+ * unsplit).  Where in_features >= 64 and num_tokens > 32, step_begin_h
+ * (nullable, room for 9) receives each split's first 64-wide step of K, then
+ * the number of steps (the last split also takes a last half step).
  */
 int pl_linear_shuffled_wide_splits(int num_tokens, int in_features, int out_features, int32_t* step_begin_h);
 int pl_linear_shuffled_wide(const void* x, int64_t ldx, int num_tokens,

@@ -12,8 +12,7 @@ namespace pl {
 namespace wgemm {
 
 constexpr int kWave = 64;
-constexpr int kBlockElems = 512;  // 16 rows x 32 k
-constexpr int kBlockBytes = 1024;
+constexpr int kBlockBytes = 1024;  // 16 rows x 32 k
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -157,6 +156,9 @@ __global__ __launch_bounds__(kStripThreads) void strip_gemm_kernel(StripArgs g) 
 // whole 128-byte lines of x per load 428 us, waves 1 x 8 (each weight block
 // loaded by one wave, not two) 369 us.  The library GEMM it replaces took 437
 // us, and 33 us to write the row-major weight it reads.
+// A last half step (K an odd multiple of 32) goes round LDS: 4112 x 2080, 2112
+// tokens, 42 us, where the strip kernel, which streams the weights once per 64
+// tokens, took 222.
 constexpr int kTileThreads = 512;
 
 // s_waitcnt vmcnt(N) as the compiler's own instruction (exp and lgkm counts
@@ -301,6 +303,22 @@ __device__ __forceinline__ void tile_gemm(const TileArgs& g) {
   for (int i = 0; i < S - 1; ++i)
     if (step + i < steps) body(step + i, buf(i), buf((i + S - 1) % S), w[i], w[(i + S - 1) % S]);
   wait_vm<0>();  // no load into LDS outlives the workgroup
+  // an odd multiple of 32: the last split takes the last 32 k, as the strip
+  // kernel does, straight into registers
+  if (g.K % 64 != 0 && split == g.splits - 1) {
+    u32x4 wt[NF];
+#pragma unroll
+    for (int n = 0; n < NF; ++n)
+      wt[n] = *reinterpret_cast<const u32x4*>(
+          (const char*)g.W + ((int64_t)min(nb0 + n, n_blocks - 1) * ksteps + ksteps - 1) * kBlockBytes + woff);
+    const char* xt = (const char*)g.x + (int64_t)t0 * g.ldx * 2 + (g.K - 32) * 2 + grp * 16;
+#pragma unroll
+    for (int m = 0; m < MF; ++m) {
+      const u32x4 a = *reinterpret_cast<const u32x4*>(xt + (int64_t)min(m * 16 + lr, g.tokens - 1 - t0) * g.ldx * 2);
+#pragma unroll
+      for (int n = 0; n < NF; ++n) acc[m][n] = mfma32<T>(wt[n], a, acc[m][n]);
+    }
+  }
 
   // lane: token lr of m tile, columns 4*grp .. +4 of n tile
 #pragma unroll
@@ -443,7 +461,7 @@ static double rows16_us(int tokens, int N, int K) {
 // these kernels leave CUs idle.
 struct Route {
   bool rows16;
-  Choice c;  // tile kernel (K % 64 == 0, more than kStripMaxTokens)
+  Choice c;  // tile kernel (K >= 64, more than kStripMaxTokens)
 };
 static Route route(int tokens, int N, int K, bool allow_split) {
   const int nb = (N + 15) / 16, mt = (tokens + 15) / 16;
@@ -454,10 +472,7 @@ static Route route(int tokens, int N, int K, bool allow_split) {
   // 10.3; a second tile of one token costs it a whole one (17 x 1902 x 12288
   // 19.5 against 18.6).
   if (tokens <= kStripMaxTokens) return {tokens >= 18 && nb * mt <= kCUs, {}};
-  // Against the strip kernel of four: one round, or two where the token tiles
-  // share the weights in an L2 (rows16_us).  64 x 1000 x 4704 10.0 us against
-  // 14.7, 2048 x 4704 10.7 against 14.6; 1902 x 4704 (476) 17.0 against 14.8.
-  if (K % 64) return {tokens <= PL_LINEAR_MAX_TOKENS && nb * mt <= (nb % 8 ? 1 : 2) * kCUs, {}};
+  if (K < 64) return {tokens <= PL_LINEAR_MAX_TOKENS, {}};  // no whole step for the tile kernel
   Choice c = choose(tokens, N, K, allow_split);
   if (tokens > PL_LINEAR_MAX_TOKENS) return {false, c};
   // Against the tile kernel, by their estimates back to back (choose's are of
@@ -501,23 +516,18 @@ static int wide(const void* x, int64_t ldx, int tokens, int K, const void* W, in
   if (!r.rows16 && r.c.splits > 1 && (ws == nullptr || ws_bytes < (size_t)r.c.splits * tokens * ldp * sizeof(float)))
     r = route(tokens, N, K, false);
   if (r.rows16) return kTakeRows16;
-  if (tokens <= kStripMaxTokens || K % 64) {
-    StripArgs g{x, W, bias, out, ldx, ldo, tokens, K, N, 0};
+  if (tokens <= kStripMaxTokens || K < 64) {
+    StripArgs g{x, W, bias, out, ldx, ldo, tokens, K, N, (tokens + 31) / 32};
     const bool narrow = N < 32 * 128;
     // two column blocks per workgroup halve the x traffic; one where that
     // would leave half the CUs idle (1000 x 2048, 17 tokens: 5.2 vs 6.0 us;
     // 24576 x 4096: 48.3 vs 46.4)
-    const int mf = tokens <= 32 ? 2 : 4, nf = narrow ? 1 : 2;
-    g.m_tiles = (tokens + 16 * mf - 1) / (16 * mf);
+    const int nf = narrow ? 1 : 2;
     const dim3 grid(g.m_tiles * (((N + 15) / 16 + nf - 1) / nf)), block(kStripThreads);
-    if (mf == 2 && narrow)
+    if (narrow)
       hipLaunchKernelGGL((strip_gemm_kernel<T, 2, 1, 2>), grid, block, 0, s, g);
-    else if (mf == 2)
-      hipLaunchKernelGGL((strip_gemm_kernel<T, 2, 2, 2>), grid, block, 0, s, g);
-    else if (narrow)
-      hipLaunchKernelGGL((strip_gemm_kernel<T, 4, 1, 2>), grid, block, 0, s, g);
     else
-      hipLaunchKernelGGL((strip_gemm_kernel<T, 4, 2, 2>), grid, block, 0, s, g);
+      hipLaunchKernelGGL((strip_gemm_kernel<T, 2, 2, 2>), grid, block, 0, s, g);
     PL_LAUNCH_CHECK("strip_gemm_kernel");
     return PL_OK;
   }
@@ -565,7 +575,7 @@ using namespace pl;
 using namespace pl::wgemm;
 
 extern "C" size_t pl_linear_shuffled_wide_workspace_size(int num_tokens, int in_features, int out_features) {
-  if (num_tokens <= kStripMaxTokens || in_features <= 0 || in_features % 64 || out_features <= 0) return 0;
+  if (num_tokens <= kStripMaxTokens || in_features < 64 || out_features <= 0) return 0;
   const Route r = route(num_tokens, out_features, in_features, true);
   const Choice& c = r.c;
   return !r.rows16 && c.splits > 1 ? (size_t)c.splits * num_tokens * split_ld(out_features) * sizeof(float) : 0;
@@ -573,7 +583,7 @@ extern "C" size_t pl_linear_shuffled_wide_workspace_size(int num_tokens, int in_
 
 extern "C" int pl_linear_shuffled_wide_splits(int num_tokens, int in_features, int out_features,
                                               int32_t* step_begin_h) {
-  if (num_tokens <= kStripMaxTokens || in_features <= 0 || in_features % 64 || out_features <= 0) return 1;
+  if (num_tokens <= kStripMaxTokens || in_features < 64 || out_features <= 0) return 1;
   const Route r = route(num_tokens, out_features, in_features, true);
   const int splits = r.rows16 ? 1 : r.c.splits;
   for (int s = 0; s <= splits && step_begin_h != nullptr; ++s)

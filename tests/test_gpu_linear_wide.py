@@ -17,7 +17,7 @@ REL = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}
 
 # Edges of the token tiles (32 .. 256 rows), of the column tiles (128 .. 384)
 # and of the K steps: 64-wide ones fewer than the buffers in flight, K not a
-# multiple of 64 (the strip kernel), K split over workgroups (few tokens, wide
+# multiple of 64, K split over workgroups (few tokens, wide
 # K), the tile shapes of many tokens.
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("tokens,n,k", [
@@ -50,6 +50,16 @@ def test_linear_wide_vs_oracle(gpu_device, dtype, tokens, n, k):
                                                (33, 4112, 3520, 4), (77, 4096, 1728, 4), (77, 8208, 4416, 2)])
 def test_uneven_splits(gpu_device, dtype, tokens, n, k, splits):
     assert _lib.load().pl_linear_shuffled_wide_splits(tokens, k, n, None) == splits
+    test_linear_wide_vs_oracle(gpu_device, dtype, tokens, n, k)
+
+
+# K an odd multiple of 32: the tile kernel's last half step, in one piece and
+# in the last of several, and a K below one step
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,n,k", [(33, 4112, 96), (65, 1000, 2080), (77, 8208, 4128), (200, 12320, 160),
+                                        (48, 24608, 1056), (2112, 6192, 96), (1000, 37, 3488), (2050, 2064, 32),
+                                        (40, 4112, 32)])
+def test_last_half_step(gpu_device, dtype, tokens, n, k):
     test_linear_wide_vs_oracle(gpu_device, dtype, tokens, n, k)
 
 

@@ -14,11 +14,12 @@ def test_every_split_has_steps(tokens):
     begin = np.zeros(9, dtype=np.int32)
     most = 0
     for n in (37, 1000, 2000, 4112, 6192):
-        for steps in range(1, 200):
-            splits = lib.pl_linear_shuffled_wide_splits(tokens, 64 * steps, n, begin.ctypes.data)
+        for k in range(64, 12800, 32):
+            steps = k // 64
+            splits = lib.pl_linear_shuffled_wide_splits(tokens, k, n, begin.ctypes.data)
             b = begin[:splits + 1]
             most = max(most, splits)
-            assert b[0] == 0 and b[-1] == steps and (np.diff(b) >= 1).all(), (tokens, n, 64 * steps, b)
+            assert b[0] == 0 and b[-1] == steps and (np.diff(b) >= 1).all(), (tokens, n, k, b)
             need = splits * tokens * -(-n // 16) * 16 * 4 if splits > 1 else 0
-            assert lib.pl_linear_shuffled_wide_workspace_size(tokens, 64 * steps, n) == need
+            assert lib.pl_linear_shuffled_wide_workspace_size(tokens, k, n) == need
     assert tokens > 128 or most == 8  # the widest split is among them
